@@ -25,12 +25,15 @@ HELD_OUT_SEED = 20240611  # generator stream of the preconditioner's held-out pa
 HBM_PEAK = 8.0e12  # B/s, MI355X
 # algorithmic bytes per cell-update of each timed kernel (fields touched once
 # per step, damping/coefficients read once per cell)
-# (k_fwd2 advances two steps per launch)
+# (k_fwd2 advances two steps per launch, k_march_fwd and k_march_adj four:
+# their figures are per cell of a launch)
 BYTES_PER_CELL = {"k_fwd": 16.0, "k_bwd": 36.0, "k_fwd2": 32.0, "k_bwd2": 72.0,
+                  "k_march_fwd": 16.0, "k_march_adj": 40.0,
                   "k_habc_fwd": 16.0, "k_habc_adj": 36.0,
                   "k_el_fwd": 52.0, "k_el_bwd": 116.0,
                   "k_fwd_batch": 16.0, "k_fwd2_batch": 32.0, "k_bwd_batch": 36.0}
-KERNEL_IDS = {"acoustic": (("k_fwd", 0), ("k_bwd", 1), ("k_fwd2", 8), ("k_bwd2", 9)),
+KERNEL_IDS = {"acoustic": (("k_fwd", 0), ("k_bwd", 1), ("k_fwd2", 8), ("k_bwd2", 9),
+                           ("k_march_fwd", 11), ("k_march_adj", 12)),
               "habc": (("k_habc_fwd", 4), ("k_habc_adj", 5)),
               "elastic": (("k_el_fwd", 2), ("k_el_bwd", 3)),
               "generator": (("k_fwd2_batch", 6), ("k_bwd_batch", 7))}  # slot 6: the batched forward, two steps per launch
@@ -781,10 +784,7 @@ def main():
           file=sys.stderr, flush=True)
     shape, tune = None, {}
     from seistorch_amd import autotune
-    if args.workload == "acoustic":
-        shape, tune = autotune.tune_acoustic(P["vp_init"], P["d"], P["w"], P["src"], P["rec"],
-                                             P["B"], P["dt"], P["h"])
-    elif args.workload == "elastic":
+    if args.workload == "elastic":
         shape, tune = autotune.tune_elastic(P["vp_init"], P["vs_init"], P["rho_init"], P["d"],
                                             P["w"], P["src"], P["rec"], P["B"], P["dt"], P["h"],
                                             src_type=("txx", "tzz"), rec_type=("vx", "vz"))

@@ -16,7 +16,7 @@
 
 #include <stdint.h>
 
-#define SEIS_ABI_VERSION 15
+#define SEIS_ABI_VERSION 16
 
 #ifdef __cplusplus
 extern "C" {
@@ -42,7 +42,9 @@ int32_t seis_abi_version(void);
 #define SEIS_KERNEL_ACOUSTIC_FWD2 8  /* k_fwd2: two forward steps per launch */
 #define SEIS_KERNEL_ACOUSTIC_BWD2 9  /* k_bwd2: two reverse steps per launch */
 #define SEIS_KERNEL_STREAM_COPY 10   /* k_stream_copy (seis_stream_copy) */
-#define SEIS_PROFILE_KERNELS 11
+#define SEIS_KERNEL_ACOUSTIC_MARCH_FWD 11 /* k_march_fwd: up to 4 forward steps per launch */
+#define SEIS_KERNEL_ACOUSTIC_MARCH_ADJ 12 /* k_march_adj: up to 4 reverse steps per launch */
+#define SEIS_PROFILE_KERNELS 13
 int seis_profile_enable(int32_t on);
 int seis_profile_collect(int32_t kernel, double* total_ms, int64_t* launches);
 
@@ -166,6 +168,42 @@ int seis_acoustic_backward(const float* vp, const float* d, const float* wavelet
                            int32_t vec_x, void* stream);
 
 /* ---------------- acoustic PML, uneven multi-model batch ------------------ */
+/* The grid rows that hold receivers: row_slot (device, int32, nz + 1) gets, per
+ * row, its number among them from the top or -1, and their count at [nz]. */
+int seis_receiver_rows(const int64_t* rec_flat, int64_t R, int64_t nz, int64_t nx,
+                       int32_t* row_slot, void* stream);
+
+/* Floats of workspace (device, 256-byte aligned) that the marching loops need
+ * for `slots` receiver rows (row_slot[nz]); adjoint: for the backward. */
+int64_t seis_acoustic_march_workspace(int64_t B, int64_t nz, int64_t nx, int32_t slots, int64_t R,
+                                      int32_t adjoint);
+
+/* seis_acoustic_forward's loop (same records, rings and snapshots, bit for
+ * bit) with up to four time steps per launch.  fields: four (B, nz, nx)
+ * buffers; final_fields (host, 2): which of them hold u^{nt} and u^{nt-1}.
+ * steps (1, 2, 4 per launch), vec_x (cells per lane 1, 2, 4; any nx), rows
+ * (grid rows per wave): 0 for automatic. */
+int seis_acoustic_march_forward(const float* vp, const float* d, const float* wavelet, int64_t nt,
+                                const int32_t* src_zx, const int64_t* rec_flat, int64_t R,
+                                const int32_t* row_slot, int32_t slots, float* rec_out,
+                                float* ring, float* snaps, int32_t snap_every, float* work,
+                                float* const* fields, int32_t* final_fields, int64_t B, int64_t nz,
+                                int64_t nx, float dt, float h, int32_t npml, int32_t multiple,
+                                int32_t steps, int32_t vec_x, int32_t rows, void* stream);
+
+/* seis_acoustic_backward's gradient with up to four reverse steps per launch
+ * (d must vanish on the undamped interior).  u, mu: four (B, nz, nx) buffers
+ * each, u[0] = u^{nt} and u[1] = u^{nt-1} (consumed); grad_part: (B, nz, nx),
+ * the shots' gradients before the factor 2c and the sum. */
+int seis_acoustic_march_backward(const float* vp, const float* d, const float* wavelet, int64_t nt,
+                                 const int32_t* src_zx, const int64_t* rec_flat, int64_t R,
+                                 const int32_t* row_slot, int32_t slots, const float* rec_grad,
+                                 const float* ring, const float* snaps, int32_t snap_every,
+                                 float* work, float* const* u, float* const* mu, float* grad_part,
+                                 float* grad, int64_t B, int64_t nz, int64_t nx, float dt, float h,
+                                 int32_t npml, int32_t multiple, int32_t steps, int32_t vec_x,
+                                 int32_t rows, void* stream);
+
 /* n independent acoustic PML problems advanced together: every time step is
  * one launch over the tiles of all instances still running (the reference
  * runs each model through its own rnn.py:178-212 loop and backward,

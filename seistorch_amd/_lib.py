@@ -38,6 +38,15 @@ SIGNATURES = {
                                               _p, _p, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _p,
                                               _p, _p, _i64, _i64, _i64, _f, _f, _i32, _i32, _i32,
                                               _i32, _i32, _p]),
+    "seis_receiver_rows": (ctypes.c_int, [_p, _i64, _i64, _i64, _p, _p]),
+    "seis_acoustic_march_workspace": (_i64, [_i64, _i64, _i64, _i32, _i64, _i32]),
+    "seis_acoustic_march_forward": (ctypes.c_int, [_p, _p, _p, _i64, _p, _p, _i64, _p, _i32, _p,
+                                                   _p, _p, _i32, _p, _p, _p, _i64, _i64, _i64, _f,
+                                                   _f, _i32, _i32, _i32, _i32, _i32, _p]),
+    "seis_acoustic_march_backward": (ctypes.c_int, [_p, _p, _p, _i64, _p, _p, _i64, _p, _i32, _p,
+                                                    _p, _p, _i32, _p, _p, _p, _p, _p, _i64, _i64,
+                                                    _i64, _f, _f, _i32, _i32, _i32, _i32, _i32,
+                                                    _p]),
     "seis_acoustic_forward_batch": (ctypes.c_int, [_i64, _p, _p, _p, _p, _p, _p, _p, _p, _p,
                                                    _p, _i32, _p, _p, _p, _p, _p, _i32, _i32, _i32,
                                                    _i32, _i32, _p]),
@@ -102,7 +111,7 @@ SIGNATURES = {
     "seis_unet_fill": (ctypes.c_int, [_p, _i64, _f, _p]),
 }
 
-ABI_VERSION = 15
+ABI_VERSION = 16
 BATCH_COLS = 23  # SEIS_BATCH_COLS: int64 columns per instance of the batch table
 
 _lock = threading.Lock()

@@ -187,6 +187,75 @@ def shared_receiver_map(rec_flat, B, nz, nx):
     return True, m.view(nz, nx)
 
 
+# Receiver rows of the marching loops: every level of a row that holds receivers
+# is written (read, in the adjoint) as a whole row, so a survey with receivers
+# on many depths (a well) keeps the loops that gather single cells.
+MARCH_CELLS = 1 << 28  # the kernels' 32-bit byte offsets within a plane
+MARCH_RING = 1 << 25   # and within the rings of a launch's time levels
+MARCH_ROWS = 8
+MARCH_ROW_SHARE = 8
+
+
+def _march_fits(B, nz, nx, need_grad, multiple):
+    """Whether the marching loops' 32-bit offsets reach and, with a gradient,
+    the interior is larger than a launch's reach."""
+    return nz * nx <= MARCH_CELLS and 2 * B * (nz + nx) <= MARCH_RING and (
+        not need_grad or (nx - 2 * NPML > 4 and nz - (1 if multiple else 2) * NPML > 4))
+
+
+def _march_rows(rec_flat, nz, nx):
+    """(row_slot int32 (nz + 1), count): the grid rows that hold receivers, or
+    None when there are too many for the marching loops."""
+    row_slot = torch.empty(nz + 1, dtype=torch.int32, device=rec_flat.device)
+    _lib.call("seis_receiver_rows", _lib.ptr(rec_flat), rec_flat.shape[0], nz, nx,
+              _lib.ptr(row_slot), _lib.stream_of(rec_flat))
+    slots = int(row_slot[nz])
+    return (row_slot, slots) if slots <= max(MARCH_ROWS, nz // MARCH_ROW_SHARE) else None
+
+
+def _march_buffers(vp, rows, R, B, n_fields, adjoint):
+    """n_fields (B, nz, nx) buffers and the workspace of a marching loop, or
+    None when they do not fit (the one- and two-step loops need fewer)."""
+    nz, nx = vp.shape
+    n = int(_lib.load().seis_acoustic_march_workspace(B, nz, nx, rows[1], R, int(adjoint)))
+    try:
+        bufs = [torch.empty((B, nz, nx), device=vp.device, dtype=torch.float32)
+                for _ in range(n_fields)]
+        return bufs, torch.empty(n, device=vp.device, dtype=torch.float32)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
+def _march_forward(bufs, work, vp, d, wavelet, src_zx, rec_flat, rows, rec, ring, snaps, K, B, dt,
+                   h, multiple, shape=(0, 0, 0)):
+    """The loop with up to four time steps per launch -> (u^nt, u^{nt-1}).
+    shape: (steps per launch, cells per lane, rows per wave), 0 automatic."""
+    nz, nx = vp.shape
+    last = torch.zeros(2, dtype=torch.int32)
+    _lib.call("seis_acoustic_march_forward", _lib.ptr(vp), _lib.ptr(d), _lib.ptr(wavelet),
+              wavelet.shape[0], _lib.ptr(src_zx), _lib.ptr(rec_flat), rec_flat.shape[0],
+              _lib.ptr(rows[0]), rows[1], _lib.ptr(rec), _lib.ptr(ring), _lib.ptr(snaps),
+              K if snaps is not None else 0, _lib.ptr(work), _lib.ptr_array(bufs),
+              _lib.ptr(last), B, nz, nx, dt, h, NPML, int(multiple), *shape, _lib.stream_of(vp))
+    return bufs[int(last[0])], bufs[int(last[1])]
+
+
+def _march_backward(bufs, work, vp, d, wavelet, src_zx, rec_flat, rows, grad_rec, ring, snaps, K,
+                    u_a, u_b, B, dt, h, multiple, shape=(0, 0, 0)):
+    """The gradient with up to four reverse steps per launch; bufs: two more
+    forward fields, four adjoint fields and the shots' gradients."""
+    nz, nx = vp.shape
+    grad = torch.empty_like(vp)
+    _lib.call("seis_acoustic_march_backward", _lib.ptr(vp), _lib.ptr(d), _lib.ptr(wavelet),
+              wavelet.shape[0], _lib.ptr(src_zx), _lib.ptr(rec_flat), rec_flat.shape[0],
+              _lib.ptr(rows[0]), rows[1], _lib.ptr(grad_rec), _lib.ptr(ring), _lib.ptr(snaps),
+              K if snaps is not None else 0, _lib.ptr(work),
+              _lib.ptr_array([u_a, u_b, bufs[0], bufs[1]]), _lib.ptr_array(bufs[2:6]),
+              _lib.ptr(bufs[6]), _lib.ptr(grad), B, nz, nx, dt, h, NPML, int(multiple), *shape,
+              _lib.stream_of(vp))
+    return grad
+
+
 class AcousticLoop(torch.autograd.Function):
     """Whole forward loop -> records (nt, R); backward = hand-written adjoint.
 
@@ -219,8 +288,14 @@ class AcousticLoop(torch.autograd.Function):
         S, rz, vx = _launch_params(B, nz, nx, shape)
         need_grad = ctx.needs_input_grad[0]
         _check_acquisition(vp, d, wavelet, src_zx, rec_flat, B, need_grad, multiple)
-        u_a = torch.empty((B, nz, nx), device=vp.device, dtype=torch.float32)
-        u_b = torch.empty_like(u_a)
+        # up to four steps per launch (the marching loops) unless the caller
+        # asks for a launch of the others: a launch shape, one step, or extra
+        # sources; the illumination keeps its own forward
+        rows = None
+        if two_step and not two_step_adjoint and all(v is None for v in shape) \
+                and _march_fits(B, nz, nx, need_grad, multiple):
+            rows = _march_rows(rec_flat, nz, nx)
+        bufs = _march_buffers(vp, rows, R, B, 4, False) if rows and illum is None else None
         rec = torch.empty((nt, R), device=vp.device, dtype=torch.float32)
         ring = None
         if need_grad and nt > 1:
@@ -236,6 +311,30 @@ class AcousticLoop(torch.autograd.Function):
             n_snap = int(_lib.load().seis_snapshot_count(nt, K))
             if n_snap > 0:
                 snaps = torch.empty((n_snap, 2, B, nz, nx), device=vp.device, dtype=torch.float32)
+        if bufs is not None:
+            u_a, u_b = _march_forward(*bufs, vp, d, wavelet, src_zx, rec_flat, rows, rec, ring,
+                                      snaps, K, B, dt, h, multiple)
+            bufs = None
+        else:
+            u_a, u_b = AcousticLoop._forward_steps(
+                vp, d, wavelet, src_zx, rec_flat, rec, ring, snaps, K, illum, two_step, extra_src,
+                extra_wav, n_extra, B, dt, h, multiple, S, rz, vx)
+        check_finite(rec)
+        if need_grad:
+            ctx.save_for_backward(vp, d, wavelet, src_zx, rec_flat)
+            ctx.state = (ring, snaps, u_a, u_b, extra_src, extra_wav, rows)
+            ctx.meta = (B, dt, h, S, K, rz, vx, bool(two_step_adjoint) and not n_extra,
+                        int(multiple))
+        return rec
+
+    @staticmethod
+    def _forward_steps(vp, d, wavelet, src_zx, rec_flat, rec, ring, snaps, K, illum, two_step,
+                       extra_src, extra_wav, n_extra, B, dt, h, multiple, S, rz, vx):
+        """One or two time steps per launch -> (u^nt, u^{nt-1})."""
+        nz, nx = vp.shape
+        nt, R = wavelet.shape[0], rec_flat.shape[0]
+        u_a = torch.empty((B, nz, nx), device=vp.device, dtype=torch.float32)
+        u_b = torch.empty_like(u_a)
         u_c = u_d = None
         if two_step and nt >= 2:
             u_c = torch.empty_like(u_a)
@@ -251,20 +350,13 @@ class AcousticLoop(torch.autograd.Function):
                   _lib.ptr(u_b),
                   _lib.ptr(u_c), _lib.ptr(u_d), B, nz, nx, dt, h, NPML, int(multiple), S, rz,
                   vx, _lib.stream_of(vp))
-        del u_c, u_d  # scratch of the two-step launches
-        check_finite(rec)
-        if need_grad:
-            ctx.save_for_backward(vp, d, wavelet, src_zx, rec_flat)
-            ctx.state = (ring, snaps, u_a, u_b, extra_src, extra_wav)
-            ctx.meta = (B, dt, h, S, K, rz, vx, bool(two_step_adjoint) and not n_extra,
-                        int(multiple))
-        return rec
+        return u_a, u_b
 
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, grad_rec):
         vp, d, wavelet, src_zx, rec_flat = ctx.saved_tensors
-        ring, snaps, u_a, u_b, extra_src, extra_wav = ctx.state
+        ring, snaps, u_a, u_b, extra_src, extra_wav, rows = ctx.state
         ctx.state = None  # the backward consumes the final forward state
         n_extra = 0 if extra_src is None else int(extra_src.shape[0])
         B, dt, h, S, K, rz, vx, two_step_adjoint, multiple = ctx.meta
@@ -273,6 +365,11 @@ class AcousticLoop(torch.autograd.Function):
         R = rec_flat.shape[0]
         G = (B + S - 1) // S
         grad_rec = grad_rec.contiguous().to(torch.float32)
+        bufs = _march_buffers(vp, rows, R, B, 7, True) if rows else None
+        if bufs is not None:
+            grad = _march_backward(*bufs, vp, d, wavelet, src_zx, rec_flat, rows, grad_rec, ring,
+                                   snaps, K, u_a, u_b, B, dt, h, multiple)
+            return (grad,) + (None,) * 15
         mu_a = torch.empty_like(u_a)
         mu_b = torch.empty_like(u_a)
         gpart = torch.empty((G, nz, nx), device=vp.device, dtype=torch.float32)
@@ -323,8 +420,10 @@ def propagate(vp, d, wavelet, src_zx, rec_flat, B, dt, h, shots_per_group=None,
     The launch shape -- shots_per_group (1, 2, 4, 8), rows_per_thread
     (1, 2, 4), vec_x (cells per lane along x: 1, 2, 4, dividing nx) --
     defaults to the autotuned values for this shape (``seistorch_amd.autotune``),
-    else to fixed defaults.  two_step runs two forward time steps per launch
-    (same results, half the forward's field traffic).  two_step_adjoint runs
+    else to fixed defaults.  With none of them given, two_step lets a launch
+    take up to four time steps (reverse steps in the adjoint; receivers on few
+    grid rows, see MARCH_ROWS); with a launch shape it runs two forward time
+    steps per launch.  Records are the same bit for bit in all of them.  two_step_adjoint runs
     two reverse steps per adjoint launch (same results up to the order of the
     gradient additions at receiver cells; at present slower than one step per
     launch: its fields of two iterations need ~250 registers per lane).
