@@ -502,6 +502,41 @@ int seis_unet_conv3x3_wgrad(const uint16_t* x, const uint16_t* dz, int32_t N, in
                             int32_t W, int32_t Cin, int32_t Cout, float* dw, float* db,
                             void* stream);
 /* dz = bf16(dy * GELU'(z)). */
+/* The convolution of the concatenation of the nearest 2x upsampling of low (N,
+ * H/2, W/2, C1; C1 a multiple of 64) and skip (N, H, W, C2), read in place. */
+int seis_unet_conv3x3_cat(const uint16_t* low, int32_t C1, const uint16_t* skip, int32_t C2,
+                          int32_t N, int32_t H, int32_t W, const uint16_t* w, const float* bias,
+                          int32_t Cout, int32_t act, uint16_t* z, uint16_t* y, void* stream);
+/* seis_unet_flip_weights for n layers in one launch: layers (host, n x 3) holds
+ * each one's offset in w (elements), Cout and Cin; the results follow each other
+ * in wt. */
+#define SEIS_UNET_MAX_LAYERS 32
+int seis_unet_flip_layers(const uint16_t* w, int32_t n, const int64_t* layers, uint16_t* wt,
+                          void* stream);
+/* seis_unet_conv3x3_wgrad with a workspace of seis_unet_wgrad_workspace floats
+ * instead of atomics (sums in a fixed order); low NULL: input x of C2 channels,
+ * else the concatenation above. */
+int64_t seis_unet_wgrad_workspace(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout);
+int seis_unet_conv3x3_wgrad_ws(const uint16_t* low, int32_t C1, const uint16_t* x, int32_t C2,
+                               const uint16_t* dz, int32_t N, int32_t H, int32_t W, int32_t Cout,
+                               float* dw, float* db, float* work, void* stream);
+/* Data gradient of a convolution (dz, Cout channels; wt from
+ * seis_unet_flip_weights) taken through the activation before it:
+ * dzp = bf16(dx * gelu'(z)), Cin channels. */
+int seis_unet_conv3x3_gelu_grad(const uint16_t* dz, int32_t N, int32_t H, int32_t W, int32_t Cout,
+                                const uint16_t* wt, int32_t Cin, const uint16_t* z, uint16_t* dzp,
+                                void* stream);
+/* Gradients of a concatenation's parts taken through their activations: low's
+ * (the 2x2 children of dout's first C1 channels summed), the skip's (dout's last
+ * C2 channels plus a quarter of dpool, the gradient of its 2x2 average pool). */
+int seis_unet_up_gelu_bwd(const float* dout, int32_t N, int32_t H, int32_t W, int32_t C1,
+                          int32_t C2, const uint16_t* z, uint16_t* dz, void* stream);
+int seis_unet_skip_gelu_bwd(const float* dout, const float* dpool, int32_t N, int32_t H, int32_t W,
+                            int32_t C1, int32_t C2, const uint16_t* z, uint16_t* dz,
+                            void* stream);
+/* Gradient of the 1x1 head over 32 channels taken through the last activation. */
+int seis_unet_head_gelu_bwd(const uint16_t* x, const float* dout, int64_t P, const float* w,
+                            const uint16_t* z, uint16_t* dz, float* dw, float* db, void* stream);
 int seis_unet_gelu_bwd(const float* dy, const uint16_t* z, int64_t n, uint16_t* dz, void* stream);
 int seis_unet_to_bf16(const float* x, int64_t n, uint16_t* y, void* stream);
 /* 2x2 average pooling and its gradient (dx = or += 0.25*dy[pixel/2]). */

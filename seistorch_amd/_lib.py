@@ -96,6 +96,18 @@ SIGNATURES = {
     "seis_unet_flip_weights": (ctypes.c_int, [_p, _i32, _i32, _p, _p]),
     "seis_unet_conv3x3_wgrad": (ctypes.c_int, [_p, _p, _i32, _i32, _i32, _i32, _i32, _p, _p,
                                                _p]),
+    "seis_unet_conv3x3_cat": (ctypes.c_int, [_p, _i32, _p, _i32, _i32, _i32, _i32, _p, _p, _i32,
+                                             _i32, _p, _p, _p]),
+    "seis_unet_flip_layers": (ctypes.c_int, [_p, _i32, _p, _p, _p]),
+    "seis_unet_wgrad_workspace": (_i64, [_i32, _i32, _i32, _i32, _i32]),
+    "seis_unet_conv3x3_wgrad_ws": (ctypes.c_int, [_p, _i32, _p, _i32, _p, _i32, _i32, _i32, _i32,
+                                                  _p, _p, _p, _p]),
+    "seis_unet_conv3x3_gelu_grad": (ctypes.c_int, [_p, _i32, _i32, _i32, _i32, _p, _i32, _p, _p,
+                                                   _p]),
+    "seis_unet_up_gelu_bwd": (ctypes.c_int, [_p, _i32, _i32, _i32, _i32, _i32, _p, _p, _p]),
+    "seis_unet_skip_gelu_bwd": (ctypes.c_int, [_p, _p, _i32, _i32, _i32, _i32, _i32, _p, _p,
+                                               _p]),
+    "seis_unet_head_gelu_bwd": (ctypes.c_int, [_p, _p, _i64, _p, _p, _p, _p, _p, _p]),
     "seis_unet_gelu_bwd": (ctypes.c_int, [_p, _p, _i64, _p, _p]),
     "seis_unet_to_bf16": (ctypes.c_int, [_p, _i64, _p, _p]),
     "seis_unet_avgpool2": (ctypes.c_int, [_p, _i32, _i32, _i32, _i32, _p, _p]),

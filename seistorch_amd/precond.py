@@ -133,6 +133,26 @@ class UNet:
             self.saved[name] = (x, z, (N, H, W))
         return y
 
+    def _conv_cat(self, low, skip, N, H, W, name, keep):
+        """_conv of the concatenation [2x upsampled low, skip], read in place
+        where the kernel can (the channels of low in whole tiles of 64)."""
+        c1, c2 = low.shape[-1], skip.shape[-1]
+        dev = low.device
+        if c1 % 64:
+            u = _bf((N, H, W, c1 + c2), dev)
+            _lib.call("seis_unet_up_concat", _lib.ptr(low), _lib.ptr(skip), N, H, W, c1, c2,
+                      _lib.ptr(u), _lib.stream_of(low))
+            return self._conv(u, N, H, W, name, keep)
+        _, _, cout = next(s for s in self.p.specs if s[0] == name)
+        y = _bf((N, H, W, cout), dev)
+        z = _bf((N, H, W, cout), dev) if keep else None
+        _lib.call("seis_unet_conv3x3_cat", _lib.ptr(low), c1, _lib.ptr(skip), c2, N, H, W,
+                  _lib.ptr(self.p.wbf16(name)), _lib.ptr(self.p.bias(name)), cout, 1,
+                  _lib.ptr(z), _lib.ptr(y), _lib.stream_of(low))
+        if keep:
+            self.saved[name] = ((low, skip), z, (N, H, W))
+        return y
+
     def forward(self, grad, model, scales, keep=False):
         """grad, model (N, H, W) FP32; scales (N, 3) FP32 = (gscale, mscale, mshift).
         Returns the (N, H, W) FP32 direction."""
@@ -158,13 +178,8 @@ class UNet:
         x = self._conv(x, N, h, w, "bota", keep)
         x = self._conv(x, N, h, w, "botb", keep)
         for l in (3, 2, 1, 0):
-            sk, h2, w2 = skips[l]
-            c1, c2 = x.shape[-1], sk.shape[-1]
-            u = _bf((N, h2, w2, c1 + c2), dev)
-            _lib.call("seis_unet_up_concat", _lib.ptr(x), _lib.ptr(sk), N, h2, w2, c1, c2,
-                      _lib.ptr(u), s)
-            h, w = h2, w2
-            x = self._conv(u, N, h, w, f"dec{l}a", keep)
+            sk, h, w = skips[l]
+            x = self._conv_cat(x, sk, N, h, w, f"dec{l}a", keep)
             x = self._conv(x, N, h, w, f"dec{l}b", keep)
         out = _f32((N, H, W), dev)
         hw, hb = self.p.head()
@@ -176,66 +191,108 @@ class UNet:
             self.saved["skip_c"] = [sk.shape[-1] for sk, _, _ in skips]
         return out
 
-    def _conv_bwd(self, name, dy, gw_arena, need_dx):
-        """dy (N,H,W,Cout) FP32 of the GELU output -> accumulates dW, db;
-        returns dx (N,H,W,Cin) FP32 if need_dx."""
+    def _wgrad(self, name, dz, gw_arena):
+        """Adds the layer's dW and db to the gradient arena (dz: bf16 gradient
+        of its pre-activation)."""
         _, cin, cout = next(s for s in self.p.specs if s[0] == name)
-        x, z, (N, H, W) = self.saved[name]
-        dev = dy.device
-        s = _lib.stream_of(dy)
-        dz = _bf((N, H, W, cout), dev)
-        _lib.call("seis_unet_gelu_bwd", _lib.ptr(dy), _lib.ptr(z), dy.numel(), _lib.ptr(dz), s)
-        _lib.call("seis_unet_conv3x3_wgrad", _lib.ptr(x), _lib.ptr(dz), N, H, W, cin, cout,
-                  _lib.ptr(self.p.weight(name, gw_arena)), _lib.ptr(self.p.bias(name, gw_arena)),
-                  s)
-        if not need_dx:
-            return None
-        wt = _bf((cin, 9 * cout), dev)
-        _lib.call("seis_unet_flip_weights", _lib.ptr(self.p.wbf16(name)), cout, cin,
-                  _lib.ptr(wt), s)
-        dx = _f32((N, H, W, cin), dev)
+        x, _, (N, H, W) = self.saved[name]
+        gw, gb = self.p.weight(name, gw_arena), self.p.bias(name, gw_arena)
+        low, skip = x if isinstance(x, tuple) else (None, x)
+        c1 = low.shape[-1] if low is not None else 0
+        n = int(_lib.load().seis_unet_wgrad_workspace(N, H, W, cin, cout))
+        work = _f32((n,), dz.device)
+        _lib.call("seis_unet_conv3x3_wgrad_ws", _lib.ptr(low), c1, _lib.ptr(skip),
+                  skip.shape[-1], _lib.ptr(dz), N, H, W, cout, _lib.ptr(gw), _lib.ptr(gb),
+                  _lib.ptr(work), _lib.stream_of(dz))
+
+    def _flip_weights(self, like):
+        """Weights of every layer's data gradient (all but the first layer's),
+        in one launch: {name: (Cin, 9 * Cout)}."""
+        layers = self.p.specs[1:]
+        host = torch.tensor([[self.p.off[name][0], cout, cin] for name, cin, cout in layers],
+                            dtype=torch.int64)
+        sizes = [cout * 9 * cin for _, cin, cout in layers]
+        wt = _bf((sum(sizes),), like.device)
+        _lib.call("seis_unet_flip_layers", _lib.ptr(self.p.bf16), len(layers), _lib.ptr(host),
+                  _lib.ptr(wt), _lib.stream_of(like))
+        return {name: w for (name, _, _), w in zip(layers, wt.split(sizes))}
+
+    def _dgrad(self, name, dz):
+        """FP32 gradient of the layer's input."""
+        _, cin, cout = next(s for s in self.p.specs if s[0] == name)
+        _, _, (N, H, W) = self.saved[name]
+        wt = self.wt[name]
+        dx = _f32((N, H, W, cin), dz.device)
         _lib.call("seis_unet_conv3x3", _lib.ptr(dz), N, H, W, cout, _lib.ptr(wt), None, cin, 0,
-                  None, None, _lib.ptr(dx), s)
+                  None, None, _lib.ptr(dx), _lib.stream_of(dz))
         return dx
+
+    def _dgrad_act(self, name, dz, before):
+        """bf16 gradient of the pre-activation of layer `before`, whose output
+        is this layer's input."""
+        _, cin, cout = next(s for s in self.p.specs if s[0] == name)
+        _, _, (N, H, W) = self.saved[name]
+        z = self.saved[before][1]
+        wt = self.wt[name]
+        out = torch.empty_like(z)
+        _lib.call("seis_unet_conv3x3_gelu_grad", _lib.ptr(dz), N, H, W, cout, _lib.ptr(wt), cin,
+                  _lib.ptr(z), _lib.ptr(out), _lib.stream_of(dz))
+        return out
+
+    def _pair_bwd(self, level, dz, grad_arena, need_dx):
+        """The two convolutions of a level (dz: gradient of the second's
+        pre-activation); returns the FP32 gradient of the level's input."""
+        self._wgrad(level + "b", dz, grad_arena)
+        dz = self._dgrad_act(level + "b", dz, level + "a")
+        self._wgrad(level + "a", dz, grad_arena)
+        return self._dgrad(level + "a", dz) if need_dx else None
 
     def backward(self, dout, grad_arena):
         """dout (N, H, W) FP32 -> parameter gradients added into grad_arena
         (same layout as the master arena; the caller zeroes it)."""
         N, H, W = self.saved["shape"]
-        dev = dout.device
         s = _lib.stream_of(dout)
         C = self.p.base
         xh = self.saved["head_in"]
-        dx = _f32((N, H, W, C), dev)
         hw, _ = self.p.head()
         gw, gb = self.p.head(grad_arena)
-        _lib.call("seis_unet_head_bwd", _lib.ptr(xh), _lib.ptr(dout.contiguous()), N * H * W, C,
-                  _lib.ptr(hw), _lib.ptr(dx), _lib.ptr(gw), _lib.ptr(gb), s)
-        dskip = [None] * 4
-        dy = dx
-        # decoder, finest level first (reverse of the forward order)
+        dout = dout.contiguous()
+        self.wt = self._flip_weights(dout)
+        dz = torch.empty_like(xh)
+        z = self.saved["dec0b"][1]
+        if C == 32:
+            _lib.call("seis_unet_head_gelu_bwd", _lib.ptr(xh), _lib.ptr(dout), N * H * W,
+                      _lib.ptr(hw), _lib.ptr(z), _lib.ptr(dz), _lib.ptr(gw), _lib.ptr(gb), s)
+        else:
+            dx = _f32((N, H, W, C), dout.device)
+            _lib.call("seis_unet_head_bwd", _lib.ptr(xh), _lib.ptr(dout), N * H * W, C,
+                      _lib.ptr(hw), _lib.ptr(dx), _lib.ptr(gw), _lib.ptr(gb), s)
+            _lib.call("seis_unet_gelu_bwd", _lib.ptr(dx), _lib.ptr(z), dx.numel(), _lib.ptr(dz),
+                      s)
+        # decoder, finest level first; the gradient of a concatenation's low
+        # part goes on through the activation that made it, the skip's part is
+        # read again by the encoder
+        below = ("dec1b", "dec2b", "dec3b", "botb")
+        cats = [None] * 4
         for l in (0, 1, 2, 3):
-            dy = self._conv_bwd(f"dec{l}b", dy, grad_arena, True)
-            du = self._conv_bwd(f"dec{l}a", dy, grad_arena, True)
-            _, _, (n_, h2, w2) = self.saved[f"dec{l}a"]
+            cats[l] = self._pair_bwd(f"dec{l}", dz, grad_arena, True)
+            _, _, (_, h, w) = self.saved[f"dec{l}a"]
             c2 = self.saved["skip_c"][l]
-            c1 = du.shape[-1] - c2
-            dlow = _f32((N, h2 // 2, w2 // 2, c1), dev)
-            dskip[l] = _f32((N, h2, w2, c2), dev)
-            _lib.call("seis_unet_up_concat_bwd", _lib.ptr(du), N, h2, w2, c1, c2,
-                      _lib.ptr(dlow), _lib.ptr(dskip[l]), 0, s)
-            dy = dlow
-        dy = self._conv_bwd("botb", dy, grad_arena, True)
-        dy = self._conv_bwd("bota", dy, grad_arena, True)
+            z = self.saved[below[l]][1]
+            dz = torch.empty_like(z)
+            _lib.call("seis_unet_up_gelu_bwd", _lib.ptr(cats[l]), N, h, w,
+                      cats[l].shape[-1] - c2, c2, _lib.ptr(z), _lib.ptr(dz), s)
+        dpool = self._pair_bwd("bot", dz, grad_arena, True)
         for l in (3, 2, 1, 0):
             # gradient of the encoder output: skip path + pooled path
-            _, _, (n_, h, w) = self.saved[f"enc{l}b"]
-            c = dskip[l].shape[-1]
-            _lib.call("seis_unet_avgpool2_bwd", _lib.ptr(dy), N, h, w, c, _lib.ptr(dskip[l]), 1,
-                      s)
-            dy = self._conv_bwd(f"enc{l}b", dskip[l], grad_arena, True)
-            dy = self._conv_bwd(f"enc{l}a", dy, grad_arena, l > 0)
-        self.saved = {}
+            z = self.saved[f"enc{l}b"][1]
+            _, h, w, c2 = z.shape
+            dz = torch.empty_like(z)
+            _lib.call("seis_unet_skip_gelu_bwd", _lib.ptr(cats[l]), _lib.ptr(dpool), N, h, w,
+                      cats[l].shape[-1] - c2, c2, _lib.ptr(z), _lib.ptr(dz), s)
+            cats[l] = None
+            dpool = self._pair_bwd(f"enc{l}", dz, grad_arena, l > 0)
+        self.saved, self.wt = {}, None
 
 
 class AdamW:
