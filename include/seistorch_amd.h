@@ -203,6 +203,30 @@ int seis_acoustic_march_backward(const float* vp, const float* d, const float* w
                                  float* grad, int64_t B, int64_t nz, int64_t nx, float dt, float h,
                                  int32_t npml, int32_t multiple, int32_t steps, int32_t vec_x,
                                  int32_t rows, void* stream);
+/* The marching loops of n independent problems together, one launch per (up to)
+ * four steps of all of them.  shape (host): n x (nz, nx, B, nt, R, receiver rows),
+ * dt_h (host): n x (dt, h); the other operands lie one problem after another, as in
+ * seis_acoustic_forward_batch, row_slot with nz + 1 entries each, fields, u, mu and
+ * grad_part with B x nz x nx.  On return fields[0] and fields[1] hold u^nt and
+ * u^{nt-1}, which the backward takes as u[0] and u[1].  work:
+ * seis_acoustic_march_batch_workspace floats (snap_every 0 without snapshots). */
+int64_t seis_acoustic_march_batch_workspace(int64_t n, const int64_t* shape, int32_t snap_every,
+                                            int32_t adjoint);
+int seis_acoustic_march_batch_forward(int64_t n, const int64_t* shape, const float* dt_h,
+                                      const float* vp, const float* d, const float* wavelet,
+                                      const int32_t* src_zx, const int64_t* rec_flat,
+                                      const int32_t* row_slot, float* rec_out, float* ring,
+                                      float* snaps, int32_t snap_every, float* work,
+                                      float* const* fields, int32_t npml, int32_t vec_x,
+                                      int32_t rows, void* stream);
+int seis_acoustic_march_batch_backward(int64_t n, const int64_t* shape, const float* dt_h,
+                                       const float* vp, const float* d, const float* wavelet,
+                                       const int32_t* src_zx, const int64_t* rec_flat,
+                                       const int32_t* row_slot, const float* rec_grad,
+                                       const float* ring, const float* snaps, int32_t snap_every,
+                                       float* work, float* const* u, float* const* mu,
+                                       float* grad_part, float* grad, int32_t npml, int32_t vec_x,
+                                       int32_t rows, void* stream);
 
 /* n independent acoustic PML problems advanced together: every time step is
  * one launch over the tiles of all instances still running (the reference

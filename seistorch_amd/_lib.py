@@ -47,6 +47,11 @@ SIGNATURES = {
                                                     _p, _p, _i32, _p, _p, _p, _p, _p, _i64, _i64,
                                                     _i64, _f, _f, _i32, _i32, _i32, _i32, _i32,
                                                     _p]),
+    "seis_acoustic_march_batch_workspace": (_i64, [_i64, _p, _i32, _i32]),
+    "seis_acoustic_march_batch_forward": (ctypes.c_int, [_i64] + [_p] * 11 + [_i32, _p, _p, _i32,
+                                          _i32, _i32, _p]),
+    "seis_acoustic_march_batch_backward": (ctypes.c_int, [_i64] + [_p] * 11 + [_i32, _p, _p, _p,
+                                           _p, _p, _i32, _i32, _i32, _p]),
     "seis_acoustic_forward_batch": (ctypes.c_int, [_i64, _p, _p, _p, _p, _p, _p, _p, _p, _p,
                                                    _p, _i32, _p, _p, _p, _p, _p, _i32, _i32, _i32,
                                                    _i32, _i32, _p]),

@@ -3,11 +3,11 @@
 The reference runs every model through its own time loop (seistorch/rnn.py:
 178-212) and boundary-saving backward (seistorch/checkpoint_new.py:146-217).
 Here many independent problems, each with its own grid, shots, time axis,
-dt, h, source and receivers, are advanced together: every time step is one
-kernel launch over the tiles of all instances still running, and the whole
-loop can be recorded into one hipGraph.  Per instance the records and the
-gradient are bit-identical to ``acoustic.propagate`` with the same launch
-shape and snapshot spacing.
+dt, h, source and receivers, are advanced together: every kernel launch takes
+up to four time steps of all instances still running (the marching loops); with
+a launch shape it is one or two, and the whole loop can be recorded into one
+hipGraph.  Per instance the records and the gradient are bit-identical to
+``acoustic.propagate`` with the same launch shape and snapshot spacing.
 
     insts = [BatchInstance(vp, d, wavelet, src_zx, rec_flat, B, dt, h), ...]
     records = propagate_batch(insts)            # list of (nt_q, R_q)
@@ -19,7 +19,8 @@ from dataclasses import dataclass
 import torch
 
 from .. import _lib
-from .acoustic import NPML, SNAP_HBM_FRACTION, SNAP_MIN_EVERY, _f, ring_len
+from .acoustic import (MARCH_ROW_SHARE, MARCH_ROWS, NPML, SNAP_HBM_FRACTION, SNAP_MIN_EVERY, _f,
+                       _march_fits, ring_len)
 
 SHAPE_COLS = 5  # nz, nx, B, nt, R
 
@@ -124,10 +125,44 @@ def _hptr(t):
     return t.data_ptr()
 
 
+def _march_rows(rec_arena, sizes):
+    """(row_slot arena, [rows with receivers]) of every instance, or None when
+    one has too many for the marching loops."""
+    at, rec, ends = 0, 0, []
+    slots = torch.empty(sum(nz + 1 for nz, *_ in sizes), dtype=torch.int32,
+                        device=rec_arena.device)
+    for nz, nx, _, _, R in sizes:
+        _lib.call("seis_receiver_rows", rec_arena.data_ptr() + 8 * rec, R, nz, nx,
+                  slots.data_ptr() + 4 * at, _lib.stream_of(rec_arena))
+        at, rec = at + nz + 1, rec + R
+        ends.append(at - 1)
+    counts = slots[torch.tensor(ends, device=slots.device)].tolist()
+    if any(c > max(MARCH_ROWS, nz // MARCH_ROW_SHARE) for c, (nz, *_) in zip(counts, sizes)):
+        return None
+    return slots, counts
+
+
+def _march_buffers(rows, sizes, fields, K, n_fields, adjoint):
+    """The instances' table (host), n_fields field arenas and the workspace of
+    the marching loops, or None when they do not fit."""
+    shape = torch.tensor([(*q, c) for q, c in zip(sizes, rows[1])], dtype=torch.int64)
+    n = int(_lib.load().seis_acoustic_march_batch_workspace(len(sizes), _hptr(shape), K,
+                                                            int(adjoint)))
+    if n < 0:
+        return None
+    f32 = dict(device=rows[0].device, dtype=torch.float32)
+    try:
+        return shape, [torch.empty(fields, **f32) for _ in range(n_fields)], torch.empty(n, **f32)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
 class _BatchLoop(torch.autograd.Function):
     @staticmethod
     def forward(ctx, vp_arena, d_arena, wav_arena, src_arena, rec_arena, sizes, dts, launch,
-                snapshot_every, use_graph, two_step=True):
+                snapshot_every, use_graph, two_step=True, march=None):
+        """march: None, or (cells per lane, rows per wave) of the marching loops, 0
+        automatic; launch is then that of the loops taken when they do not fit."""
         S, rz, vx = launch
         dev = vp_arena.device
         need_grad = ctx.needs_input_grad[0]
@@ -140,24 +175,39 @@ class _BatchLoop(torch.autograd.Function):
         n = len(sizes)
         f32 = dict(device=dev, dtype=torch.float32)
         rec = torch.empty(lay.total["out"], **f32)
-        u_a = torch.empty(lay.total["field"], **f32)
-        u_b = torch.empty_like(u_a)
-        # two steps per launch need the third and fourth field arenas
-        u_c, u_d = (torch.empty_like(u_a), torch.empty_like(u_a)) if two_step else (None, None)
         ring = torch.empty(lay.total["ring"], **f32) if need_grad and lay.total["ring"] else None
         snaps = torch.empty(lay.total["snap"], **f32) if K > 0 and lay.total["snap"] else None
-        table = torch.empty(n * _lib.BATCH_COLS, device=dev, dtype=torch.int64)
-        _lib.call("seis_acoustic_forward_batch", n, _hptr(shape), _hptr(dt_h), _lib.ptr(vp_arena),
-                  _lib.ptr(d_arena), _lib.ptr(wav_arena), _lib.ptr(src_arena),
-                  _lib.ptr(rec_arena), _lib.ptr(rec), _lib.ptr(ring), _lib.ptr(snaps),
-                  K if snaps is not None else 0, _lib.ptr(u_a), _lib.ptr(u_b), _lib.ptr(u_c),
-                  _lib.ptr(u_d), _lib.ptr(table), NPML, S, rz, vx, int(use_graph),
-                  _lib.stream_of(vp_arena))
-        del u_c, u_d
+        K = K if snaps is not None else 0
+        rows = _march_rows(rec_arena, sizes) if march is not None and two_step and all(
+            _march_fits(B, nz, nx, need_grad, False) for nz, nx, B, _, _ in sizes) else None
+        bufs = _march_buffers(rows, sizes, lay.total["field"], K, 4, False) if rows else None
+        table = None
+        if bufs is not None:
+            mshape, fields, work = bufs
+            _lib.call("seis_acoustic_march_batch_forward", n, _hptr(mshape), _hptr(dt_h),
+                      _lib.ptr(vp_arena), _lib.ptr(d_arena), _lib.ptr(wav_arena),
+                      _lib.ptr(src_arena), _lib.ptr(rec_arena), _lib.ptr(rows[0]), _lib.ptr(rec),
+                      _lib.ptr(ring), _lib.ptr(snaps), K, _lib.ptr(work), _lib.ptr_array(fields),
+                      NPML, *march, _lib.stream_of(vp_arena))
+            u_a, u_b = fields[:2]
+            del bufs, fields, work
+        else:
+            u_a = torch.empty(lay.total["field"], **f32)
+            u_b = torch.empty_like(u_a)
+            # two steps per launch need the third and fourth field arenas
+            u_c, u_d = (torch.empty_like(u_a), torch.empty_like(u_a)) if two_step else (None, None)
+            table = torch.empty(n * _lib.BATCH_COLS, device=dev, dtype=torch.int64)
+            _lib.call("seis_acoustic_forward_batch", n, _hptr(shape), _hptr(dt_h),
+                      _lib.ptr(vp_arena), _lib.ptr(d_arena), _lib.ptr(wav_arena),
+                      _lib.ptr(src_arena), _lib.ptr(rec_arena), _lib.ptr(rec), _lib.ptr(ring),
+                      _lib.ptr(snaps), K, _lib.ptr(u_a), _lib.ptr(u_b), _lib.ptr(u_c),
+                      _lib.ptr(u_d), _lib.ptr(table), NPML, S, rz, vx, int(use_graph),
+                      _lib.stream_of(vp_arena))
+            del u_c, u_d
         if need_grad:
             ctx.save_for_backward(vp_arena, d_arena, wav_arena, src_arena, rec_arena)
-            ctx.state = (ring, snaps, u_a, u_b, table)
-            ctx.meta = (sizes, dts, launch, K if snaps is not None else 0, use_graph, lay)
+            ctx.state = (ring, snaps, u_a, u_b, table, rows)
+            ctx.meta = (sizes, dts, launch, K, use_graph, lay, march)
         # one output per instance, so the backward receives each cotangent once
         return tuple(rec[o:o + nt * R].view(nt, R)
                      for o, (_, _, _, nt, R) in zip(lay.off["out"], sizes))
@@ -167,22 +217,38 @@ class _BatchLoop(torch.autograd.Function):
     def backward(ctx, *grad_recs):
         grad_rec = torch.cat([g.reshape(-1) for g in grad_recs])
         vp_arena, d_arena, wav_arena, src_arena, rec_arena = ctx.saved_tensors
-        ring, snaps, u_a, u_b, table = ctx.state
+        ring, snaps, u_a, u_b, table, rows = ctx.state
         ctx.state = None  # the backward consumes the final forward state
-        sizes, dts, (S, rz, vx), K, use_graph, lay = ctx.meta
+        sizes, dts, (S, rz, vx), K, use_graph, lay, march = ctx.meta
         shape, dt_h = _host_tables(sizes, dts)
+        grad_rec = grad_rec.contiguous().float()
+        grad = torch.empty_like(vp_arena)
+        # two more forward fields, four adjoint fields, the shots' gradients
+        bufs = _march_buffers(rows, sizes, lay.total["field"], K, 7, True) if rows else None
+        if bufs is not None:
+            mshape, fields, work = bufs
+            _lib.call("seis_acoustic_march_batch_backward", len(sizes), _hptr(mshape),
+                      _hptr(dt_h), _lib.ptr(vp_arena), _lib.ptr(d_arena), _lib.ptr(wav_arena),
+                      _lib.ptr(src_arena), _lib.ptr(rec_arena), _lib.ptr(rows[0]),
+                      _lib.ptr(grad_rec), _lib.ptr(ring), _lib.ptr(snaps), K, _lib.ptr(work),
+                      _lib.ptr_array([u_a, u_b, *fields[:2]]), _lib.ptr_array(fields[2:6]),
+                      _lib.ptr(fields[6]), _lib.ptr(grad), NPML, *march,
+                      _lib.stream_of(vp_arena))
+            return (grad,) + (None,) * 11
+        if table is None:
+            table = torch.empty(len(sizes) * _lib.BATCH_COLS, device=u_a.device,
+                                dtype=torch.int64)
         mu_a = torch.empty_like(u_a)
         mu_b = torch.empty_like(u_a)
         gpart = torch.empty(lay.total["gpart"], device=u_a.device, dtype=torch.float32)
-        grad = torch.empty_like(vp_arena)
         _lib.call("seis_acoustic_backward_batch", len(sizes), _hptr(shape), _hptr(dt_h),
                   _lib.ptr(vp_arena), _lib.ptr(d_arena), _lib.ptr(wav_arena),
                   _lib.ptr(src_arena), _lib.ptr(rec_arena),
-                  _lib.ptr(grad_rec.contiguous().float()), _lib.ptr(ring), _lib.ptr(snaps), K,
+                  _lib.ptr(grad_rec), _lib.ptr(ring), _lib.ptr(snaps), K,
                   _lib.ptr(u_a), _lib.ptr(u_b), _lib.ptr(mu_a), _lib.ptr(mu_b), _lib.ptr(gpart),
                   _lib.ptr(grad), _lib.ptr(table), NPML, S, rz, vx, int(use_graph),
                   _lib.stream_of(vp_arena))
-        return (grad,) + (None,) * 10
+        return (grad,) + (None,) * 11
 
 
 def _launch_params(sizes, shape):
@@ -200,9 +266,11 @@ def propagate_batch(insts, shots_per_group=None, rows_per_thread=None, vec_x=Non
     shots_per_group / rows_per_thread / vec_x: launch shape shared by the whole
     batch (None: tuned or default; vec_x must divide every nx).  snapshot_every:
     one spacing for all instances (None automatic, 0 ring only).  use_graph:
-    record the time loop into one hipGraph (False: direct launches).
-    two_step: the forward advances two time steps per launch (two more field
-    arenas; records, rings and snapshots bit-identical to one step per launch).
+    record the time loop into one hipGraph (False: direct launches), where a
+    launch takes one or two steps.  two_step: launches take up to four time
+    steps, or, with a launch shape or receivers on many grid rows, two in the
+    forward (two more field arenas; records, rings and snapshots bit-identical
+    to one step per launch).
     """
     insts = list(insts)
     if not insts:
@@ -214,7 +282,9 @@ def propagate_batch(insts, shots_per_group=None, rows_per_thread=None, vec_x=Non
     sizes = [(int(it.vp.shape[0]), int(it.vp.shape[1]), int(it.B), int(it.wavelet.shape[0]),
               int(it.rec_flat.shape[0])) for it in insts]
     dts = [(_f(it.dt), _f(it.h)) for it in insts]
-    launch = _launch_params(sizes, (shots_per_group, rows_per_thread, vec_x))
+    shape = (shots_per_group, rows_per_thread, vec_x)
+    launch = _launch_params(sizes, shape)
+    march = (0, 0) if all(v is None for v in shape) else None
     vp_arena = torch.cat([v.reshape(-1) for v in vps])
     with torch.no_grad():
         d_arena = torch.cat([it.d.reshape(-1).float() for it in insts])
@@ -222,4 +292,5 @@ def propagate_batch(insts, shots_per_group=None, rows_per_thread=None, vec_x=Non
         src_arena = torch.cat([it.src_zx.reshape(-1) for it in insts])
         rec_arena = torch.cat([it.rec_flat.reshape(-1) for it in insts])
     return list(_BatchLoop.apply(vp_arena, d_arena, wav_arena, src_arena, rec_arena, sizes,
-                                 dts, launch, snapshot_every, bool(use_graph), bool(two_step)))
+                                 dts, launch, snapshot_every, bool(use_graph), bool(two_step),
+                                 march))
