@@ -424,6 +424,19 @@ int seis_elastic_forward(const float* coef, const float* wavelet, int64_t nt,
                          int32_t illum_field, float* const* fields, float* const* scratch,
                          int64_t B, int64_t nz, int64_t nx, float dt, float h, int32_t npml,
                          int32_t multiple, int32_t shots_per_group, void* stream);
+/* The forward loop with up to three time steps per launch (steps, vec_x 1 or 2,
+ * rows per wave: 0 automatic); results as seis_elastic_forward with scratch.
+ * row_slot and slots: seis_receiver_rows; rec_mask: the fields of the channels;
+ * work: seis_elastic_march_workspace floats. */
+int64_t seis_elastic_march_workspace(int64_t B, int64_t nx, int32_t slots, int64_t R);
+int seis_elastic_march_forward(const float* coef, const float* wavelet, int64_t nt,
+                               const int32_t* src_zx, int32_t src_mask, const int64_t* rec_flat,
+                               int64_t R, const int32_t* rec_field, int32_t rec_mask, int32_t nch,
+                               const int32_t* row_slot, int32_t slots, float* rec_out, float* ring,
+                               float* snaps, int32_t snap_every, float* work,
+                               float* const* fields, float* const* scratch, int64_t B, int64_t nz,
+                               int64_t nx, float dt, float h, int32_t npml, int32_t multiple,
+                               int32_t steps, int32_t vec_x, int32_t rows, void* stream);
 
 /* Adjoint of seis_elastic_forward with boundary-saving reconstruction
  * (replaces seistorch/checkpoint.py:108-230 and elastic.py:39-122 with the

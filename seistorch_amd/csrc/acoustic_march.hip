@@ -3,6 +3,7 @@
 // rings and snapshots written and read by the launches themselves.
 #include "common.h"
 #include "march.h"
+#include "march_rows.h"
 #include "seistorch_amd.h"
 #include "tiles.h"
 
@@ -37,11 +38,6 @@ __global__ __launch_bounds__(256) void k_mark_rows(const int64_t* __restrict__ r
   if (t < R) row_slot[(rec[t] % plane) / nx] = 0;
 }
 
-__global__ __launch_bounds__(256) void k_fill_i32(int32_t* __restrict__ p, int64_t n, int32_t v) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = v;
-}
-
 // Marked rows numbered from the top, their count in row_slot[nz]; one wave.
 __global__ __launch_bounds__(64) void k_number_rows(int32_t* __restrict__ row_slot, int nz) {
   int base = 0;
@@ -53,22 +49,6 @@ __global__ __launch_bounds__(64) void k_number_rows(int32_t* __restrict__ row_sl
     base += __popcll(m);
   }
   if (threadIdx.x == 0) row_slot[nz] = base;
-}
-
-// Receiver t's cell in the (slots, B, nx) rows; with head/next, the receivers
-// of one cell are chained for the adjoint's sources.
-__global__ __launch_bounds__(256) void k_row_cells(const int64_t* __restrict__ rec, int64_t R,
-                                                   int64_t plane, int nx, int B,
-                                                   const int32_t* __restrict__ row_slot,
-                                                   int64_t* __restrict__ cell,
-                                                   int32_t* __restrict__ head,
-                                                   int32_t* __restrict__ next) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= R) return;
-  const int64_t b = rec[t] / plane, i = rec[t] - b * plane;
-  const int64_t c = ((int64_t)row_slot[i / nx] * B + b) * nx + i % nx;
-  if (cell) cell[t] = c;
-  if (head) next[t] = atomicExch(head + c, (int32_t)t);
 }
 
 // Work beside the march of one launch: the records of the previous launch's
@@ -114,23 +94,6 @@ __device__ __forceinline__ void fill_sources(const Sources& so, int block) {
 __global__ __launch_bounds__(kThreads) void k_gather(Gather ga) { gather_records(ga, blockIdx.x); }
 __global__ __launch_bounds__(kThreads) void k_sources(Sources so) { fill_sources(so, blockIdx.x); }
 
-// XCD-aware block order, as tiles.h: each XCD takes a contiguous range.
-__device__ __forceinline__ int xcd_block(int per) {
-  const int w = blockIdx.x;
-  return (w % kXcds) * per + w / kXcds;
-}
-
-__device__ __forceinline__ bool march_unit(const Split& sp, int B, int blk, int& strip, int& seg,
-                                           int& b) {
-  const int64_t unit = (int64_t)blk * kWavesPerBlock +
-                       __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-  const int64_t row = unit / sp.group, row2 = row / sp.strips;
-  strip = (int)(row - row2 * sp.strips);
-  seg = (int)(row2 % sp.segs);
-  b = (int)(row2 / sp.segs) * sp.group + (int)(unit - row * sp.group);
-  return b < B;
-}
-
 // The kernels take one struct, so that its constant-memory copy is at the
 // start of the kernel's arguments.
 struct FwdLaunch {
@@ -144,11 +107,6 @@ struct AdjLaunch {
   Sources so;
   int per;
 };
-
-template <typename P>
-__device__ __forceinline__ Const<P> launch_params() {
-  return (Const<P>)__builtin_amdgcn_kernarg_segment_ptr();
-}
 
 template <int T, int VX>
 __global__ __launch_bounds__(kThreads) void k_march_fwd(FwdLaunch a) {
@@ -269,25 +227,6 @@ __global__ __launch_bounds__(256) void k_march_grad(const float* __restrict__ vp
   grad[i] = 2.0f * vp[i] * s;
 }
 
-__global__ __launch_bounds__(256) void k_zero(float* __restrict__ p, int64_t n) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = 0.0f;
-}
-
-__global__ __launch_bounds__(256) void k_copy(const float* __restrict__ a, float* __restrict__ b,
-                                              int64_t n) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) b[t] = a[t];
-}
-
-inline unsigned blocks_of(int64_t n) { return (unsigned)((n + 255) / 256); }
-
-int zero(float* p, int64_t n, hipStream_t s) {
-  k_zero<<<blocks_of(n), 256, 0, s>>>(p, n);
-  SEIS_CHECK_LAUNCH();
-  return 0;
-}
-
 // Shots whose waves run side by side on the same strips.  Eight share the
 // coefficient rows in L2 while neighbouring segments still find each other's
 // halo rows in the last-level cache: 64 shots of 900 x 2500, 10^9 cell updates
@@ -390,8 +329,6 @@ Plan make_plan(int64_t n, int wide, int32_t steps, int32_t vec_x, int32_t rows) 
   return p;
 }
 
-inline int64_t pad64(int64_t n) { return (n + 63) / 64 * 64; }
-
 // Workspace (in floats): coefficient planes, two sets of receiver rows, the
 // receivers' cells (forward) or chains (adjoint).
 struct Work {
@@ -421,8 +358,6 @@ Work carve(float* base, int64_t B, int64_t nz, int64_t nx, int64_t slots, int64_
   w.total = o;
   return w;
 }
-
-int aux_blocks(int64_t n) { return (int)std::min<int64_t>((n + kThreads - 1) / kThreads, 512); }
 
 int check_march(int64_t B, int64_t nz, int64_t nx, float dt, float h, int64_t nt, int64_t R,
                 int32_t npml, int32_t slots, const int32_t* row_slot, int32_t steps,
@@ -744,11 +679,6 @@ void add_item(std::vector<Item>& items, Round& r, Item it, int64_t blocks) {
   r.aux_blocks += it.aux.blocks;
   ++r.n;
   items.push_back(it);
-}
-
-int64_t split_blocks(const Split& sp, int64_t B) {
-  const int64_t units = (int64_t)sp.strips * sp.segs * sp.group * ((B + sp.group - 1) / sp.group);
-  return (units + kWavesPerBlock - 1) / kWavesPerBlock;
 }
 
 template <typename Item, typename K>

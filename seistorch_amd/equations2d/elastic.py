@@ -25,6 +25,9 @@ from .acoustic import check_finite
 from .utils import restore_boundaries
 
 NPML = 49
+# the marching forward's 32-bit byte offsets: cells of a grid, ring floats of a step
+MARCH_CELLS = 1 << 26
+MARCH_RING = 1 << 25
 N = 1
 FIELDS = ("vx", "vz", "txx", "tzz", "txz")
 
@@ -117,6 +120,35 @@ def _mask(names):
     return m
 
 
+def _march_work(rec_flat, B, nz, nx):
+    """(rows, workspace) of the marching forward, or None where its 32-bit
+    offsets do not reach, receivers lie on many grid rows or memory is short."""
+    from .acoustic import _march_rows
+    if nz * nx > MARCH_CELLS or 2 * 5 * B * (nz + nx) > MARCH_RING:
+        return None
+    rows = _march_rows(rec_flat, nz, nx)
+    if rows is None:
+        return None
+    n = int(_lib.load().seis_elastic_march_workspace(B, nx, rows[1], rec_flat.shape[0]))
+    try:
+        return rows, torch.empty(n, device=rec_flat.device, dtype=torch.float32)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
+def _march_forward(rows, work, cf, wavelet, src_zx, src_mask, rec_flat, rf, rec_mask, nch, rec,
+                   ring, snaps, K, fields, scratch, B, dt, h, multiple, shape=(0, 0, 0)):
+    """The forward loop with up to three steps per launch.  shape: (steps per
+    launch, cells per lane, rows per wave), 0 automatic."""
+    nz, nx = cf.shape[-2:]
+    _lib.call("seis_elastic_march_forward", _lib.ptr(cf), _lib.ptr(wavelet), wavelet.shape[0],
+              _lib.ptr(src_zx), src_mask, _lib.ptr(rec_flat), rec_flat.shape[0], _lib.ptr(rf),
+              rec_mask, nch, _lib.ptr(rows[0]), rows[1], _lib.ptr(rec), _lib.ptr(ring),
+              _lib.ptr(snaps), K if snaps is not None else 0, _lib.ptr(work),
+              _lib.ptr_array(fields), _lib.ptr_array(scratch), B, nz, nx, dt, h, NPML,
+              int(multiple), *shape, _lib.stream_of(cf))
+
+
 class ElasticLoop(torch.autograd.Function):
     """Whole elastic loop -> records (nt, R, nch); backward -> (dvp, dvs, drho)."""
 
@@ -132,6 +164,7 @@ class ElasticLoop(torch.autograd.Function):
         nz, nx = vp.shape
         nt = wavelet.shape[0]
         R = rec_flat.shape[0]
+        marching = fused and illum is None and shots_per_group is None
         if shots_per_group is None:
             from .. import autotune
             shots_per_group = autotune.lookup("elastic", B, vp.shape[0], vp.shape[1])
@@ -157,12 +190,19 @@ class ElasticLoop(torch.autograd.Function):
             if n_snap > 0:
                 snaps = torch.empty((n_snap, 5, B, nz, nx), device=vp.device)
         scratch = [torch.empty_like(fields[0]) for _ in range(5)] if fused else None
-        _lib.call("seis_elastic_forward", _lib.ptr(cf), _lib.ptr(wavelet), nt, _lib.ptr(src_zx),
-                  _mask(src_type), _lib.ptr(rec_flat), R, _lib.ptr(rf), nch, _lib.ptr(rec),
-                  _lib.ptr(ring), _lib.ptr(snaps), K, _lib.ptr(illum),
-                  FIELDS.index(src_type[-1]), _lib.ptr_array(fields),
-                  _lib.ptr_array(scratch) if fused else None, B, nz, nx, dt, h, NPML,
-                  int(multiple), S, _lib.stream_of(vp))
+        # up to three steps per launch; a launch shape and the illumination keep one
+        march = _march_work(rec_flat, B, nz, nx) if marching else None
+        if march is not None:
+            _march_forward(*march, cf, wavelet, src_zx, _mask(src_type), rec_flat, rf,
+                           _mask(rec_type), nch, rec, ring, snaps, K, fields, scratch, B, dt, h,
+                           multiple)
+        else:
+            _lib.call("seis_elastic_forward", _lib.ptr(cf), _lib.ptr(wavelet), nt,
+                      _lib.ptr(src_zx), _mask(src_type), _lib.ptr(rec_flat), R, _lib.ptr(rf), nch, _lib.ptr(rec),
+                      _lib.ptr(ring), _lib.ptr(snaps), K, _lib.ptr(illum),
+                      FIELDS.index(src_type[-1]), _lib.ptr_array(fields),
+                      _lib.ptr_array(scratch) if fused else None, B, nz, nx, dt, h, NPML,
+                      int(multiple), S, _lib.stream_of(vp))
         del scratch  # ping-pong buffers of the fused steps
         check_finite(rec)
         if need_grad:
