@@ -314,6 +314,32 @@ int seis_habc_backward(const float* vp, const float* b, const float* wavelet, in
                        float* l_c, float* grad_part, float* grad, int64_t B, int64_t nz,
                        int64_t nx, float dt, float h, int32_t npml, int32_t multiple,
                        int32_t shots_per_group, void* stream);
+/* The HABC loops with up to four steps per launch away from the edges (Core) and
+ * one at a time in the frame around it; grids that seis_habc_march_fits accepts.
+ * row_slot (nz + 1) and slots = row_slot[nz]: the rows of Core and of the three cells
+ * around it with receivers, from seis_habc_core_rows.  fields: five buffers, final_fields (host) the indices of
+ * u^nt and u^{nt-1}; u: four (u^nt, u^{nt-1} first), lam: five, grad_core: B planes,
+ * grad_part: one per shot group.  vec_x, rows: cells per lane and rows per wave of
+ * Core, 0 automatic.  work: seis_habc_march_workspace floats. */
+int32_t seis_habc_march_fits(int64_t nz, int64_t nx);
+int seis_habc_core_rows(const int64_t* rec_flat, int64_t R, int64_t nz, int64_t nx,
+                        int32_t* row_slot, void* stream);
+int64_t seis_habc_march_workspace(int64_t B, int64_t nz, int64_t nx, int32_t slots, int64_t R);
+int seis_habc_march_forward(const float* vp, const float* b, const float* wavelet, int64_t nt,
+                            const int32_t* src_zx, const int64_t* rec_flat, int64_t R,
+                            const int32_t* row_slot, int32_t slots, float* rec_out, float* ring,
+                            float* snaps, int32_t snap_every, float* work, float* const* fields,
+                            int32_t* final_fields, int64_t B, int64_t nz, int64_t nx, float dt,
+                            float h, int32_t npml, int32_t multiple, int32_t shots_per_group,
+                            int32_t vec_x, int32_t rows, void* stream);
+int seis_habc_march_backward(const float* vp, const float* b, const float* wavelet, int64_t nt,
+                             const int32_t* src_zx, const int64_t* rec_flat, int64_t R,
+                             const int32_t* row_slot, int32_t slots, const float* rec_grad,
+                             const float* ring, const float* snaps, int32_t snap_every,
+                             float* work, float* const* u, float* const* lam, float* grad_core,
+                             float* grad_part, float* grad, int64_t B, int64_t nz, int64_t nx,
+                             float dt, float h, int32_t npml, int32_t multiple,
+                             int32_t shots_per_group, int32_t vec_x, int32_t rows, void* stream);
 
 /* ---------------- variable-density acoustic equation (HABC) --------------- */
 /* One step of seistorch/equations2d/acoustic_rho_habc.py:31-57 (blend = 1:

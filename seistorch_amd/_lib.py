@@ -77,6 +77,15 @@ SIGNATURES = {
     "seis_habc_backward": (ctypes.c_int, [_p, _p, _p, _i64, _p, _p, _i64, _p, _p, _p, _i32, _p,
                                           _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _f, _f, _i32,
                                           _i32, _i32, _p]),
+    "seis_habc_march_fits": (_i32, [_i64, _i64]),
+    "seis_habc_core_rows": (ctypes.c_int, [_p, _i64, _i64, _i64, _p, _p]),
+    "seis_habc_march_workspace": (_i64, [_i64, _i64, _i64, _i32, _i64]),
+    "seis_habc_march_forward": (ctypes.c_int, [_p, _p, _p, _i64, _p, _p, _i64, _p, _i32, _p, _p,
+                                _p, _i32, _p, _p, _p, _i64, _i64, _i64, _f, _f, _i32, _i32, _i32,
+                                _i32, _i32, _p]),
+    "seis_habc_march_backward": (ctypes.c_int, [_p, _p, _p, _i64, _p, _p, _i64, _p, _i32, _p, _p,
+                                 _p, _i32, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _f, _f,
+                                 _i32, _i32, _i32, _i32, _i32, _p]),
     "seis_elastic_coefficients": (ctypes.c_int, [_p, _p, _p, _p, _p, _i64, _i64, _f, _f, _p]),
     "seis_elastic_stage": (ctypes.c_int, [_i32, _p, _p, _f, _i32, _i32, _i32, _i32, _i64, _i64,
                                           _i64, _f, _f, _i32, _p]),

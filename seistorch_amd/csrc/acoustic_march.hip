@@ -17,38 +17,12 @@ using seis::tiles::kXcds;
 
 namespace {
 
-// c^2, A and B of the damped update, once per loop.
-__global__ __launch_bounds__(256) void k_coefs(const float* __restrict__ vp,
-                                               const float* __restrict__ d, int64_t plane,
-                                               TimeConsts k, float* __restrict__ c2,
-                                               float* __restrict__ A, float* __restrict__ Bc) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= plane) return;
-  const float c = vp[i], dd = d[i];
-  c2[i] = c * c;
-  A[i] = 1.0f / (k.idt2 + dd * k.idt);
-  Bc[i] = k.idt2 - dd * k.idt;
-}
-
 // row_slot[z] = 0 for every row that holds a receiver of any shot (-1 before).
 __global__ __launch_bounds__(256) void k_mark_rows(const int64_t* __restrict__ rec, int64_t R,
                                                    int64_t plane, int nx,
                                                    int32_t* __restrict__ row_slot) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < R) row_slot[(rec[t] % plane) / nx] = 0;
-}
-
-// Marked rows numbered from the top, their count in row_slot[nz]; one wave.
-__global__ __launch_bounds__(64) void k_number_rows(int32_t* __restrict__ row_slot, int nz) {
-  int base = 0;
-  for (int z0 = 0; z0 < nz; z0 += 64) {
-    const int z = z0 + (int)threadIdx.x;
-    const bool on = z < nz && row_slot[z] >= 0;
-    const unsigned long long m = __ballot(on);
-    if (on) row_slot[z] = base + __popcll(m & ((1ull << threadIdx.x) - 1));
-    base += __popcll(m);
-  }
-  if (threadIdx.x == 0) row_slot[nz] = base;
 }
 
 // Work beside the march of one launch: the records of the previous launch's
@@ -61,14 +35,6 @@ struct Gather {
   int levels, blocks;    // blocks of 256 threads, after the march's
 };
 
-struct Sources {
-  float* rows;           // (levels, row_cells) of the next launch
-  const int32_t *head, *next;
-  int64_t R, row_cells;
-  const float* rgrad;    // row of the first level; the next level's precedes it
-  int levels, blocks;
-};
-
 __device__ __forceinline__ void gather_records(const Gather& ga, int block) {
   const int64_t n = ga.R * ga.levels;
   for (int64_t i = (int64_t)block * kThreads + threadIdx.x; i < n;
@@ -78,22 +44,7 @@ __device__ __forceinline__ void gather_records(const Gather& ga, int block) {
   }
 }
 
-__device__ __forceinline__ void fill_sources(const Sources& so, int block) {
-  for (int64_t c = (int64_t)block * kThreads + threadIdx.x; c < so.row_cells;
-       c += (int64_t)so.blocks * kThreads) {
-    const int32_t h = so.head[c];
-    for (int lev = 0; lev < so.levels; ++lev) {
-      const float* rg = so.rgrad - (int64_t)lev * so.R;
-      float s = 0.0f;
-      for (int32_t t = h; t >= 0; t = so.next[t]) s += rg[t];
-      so.rows[lev * so.row_cells + c] = s;
-    }
-  }
-}
-
 __global__ __launch_bounds__(kThreads) void k_gather(Gather ga) { gather_records(ga, blockIdx.x); }
-__global__ __launch_bounds__(kThreads) void k_sources(Sources so) { fill_sources(so, blockIdx.x); }
-
 // The kernels take one struct, so that its constant-memory copy is at the
 // start of the kernel's arguments.
 struct FwdLaunch {
@@ -227,13 +178,6 @@ __global__ __launch_bounds__(256) void k_march_grad(const float* __restrict__ vp
   grad[i] = 2.0f * vp[i] * s;
 }
 
-// Shots whose waves run side by side on the same strips.  Eight share the
-// coefficient rows in L2 while neighbouring segments still find each other's
-// halo rows in the last-level cache: 64 shots of 900 x 2500, 10^9 cell updates
-// per second of the adjoint with groups of 1 / 4 / 8 / 16 / 64: 335 / 393 /
-// 399 / 375 / 343; of the forward 887 / 922 / 937 / 921 / 836.
-constexpr int kShotGroup = 8;
-
 #define SEIS_MARCH_CASES(F) \
   F(1, 1) F(1, 2) F(1, 4) F(2, 1) F(2, 2) F(2, 4) F(4, 1) F(4, 2) F(4, 4)
 
@@ -284,50 +228,9 @@ int launch_adj(int T, int VX, const Coefs& cf, const AdjLevels& f, const int32_t
   return 0;
 }
 
-constexpr int kMaxT = kMaxSteps;
 // ring floats of one time level: those of a launch's levels are one buffer,
 // whose offsets stay below kRowOut bytes
 constexpr int64_t kMaxRing = (int64_t)1 << 25;
-
-// Steps of the next launch when `left` remain to the next boundary: the
-// remainder first, so that the launch that ends at the boundary takes at
-// least two steps (and can write both fields of a snapshot) unless left == 1.
-inline int next_steps(int64_t left, int max_t) {
-  const int64_t r = left % max_t;
-  if (r == 0) return max_t;
-  return r >= 2 ? 2 : 1;
-}
-
-inline int widest(int64_t nx) { return nx % 4 == 0 ? 4 : nx % 2 == 0 ? 2 : 1; }
-
-struct Plan {
-  int vx_f, vx_a, rows_f, rows_a, t_f, t_a;
-};
-
-// Launch shape; 0 = automatic.  Four steps per launch at every size (two were
-// slower throughout).  Wide lanes on long segments recompute least, narrow
-// lanes on short segments give the most waves: the lines are where the better
-// one changed in microseconds per step, forward / adjoint, (cells per lane,
-// rows): 164 x 164 x 1 shot (1, 4) 3.6 / 5.4, (1, 8) 3.8 / 6.7; 300 x 500 x 8
-// (1, 8) 4.4 / 9.0, (1, 12) 4.7 / 8.8, (2, 8) 4.5 / 9.1; 900 x 2500 x 2 (1, 16)
-// 7.6 / 14.4, (2, 16) 7.5 / 15.5; x 8 (4, 16) 23.6 and (2, 12) 57 of the adjoint
-// against (4, 16) 60; x 64 (4, 32) 143 / 279, (2, 32) 156 / 284, (4, 16) 148 /
-// 318.
-// n cells of all shots, `wide` the widest lanes that divide the grid.
-Plan make_plan(int64_t n, int wide, int32_t steps, int32_t vec_x, int32_t rows) {
-  Plan p;
-  p.t_f = p.t_a = steps ? steps : 4;
-  if (n < 300000) { p.vx_f = p.vx_a = 1; p.rows_f = p.rows_a = 4; }
-  else if (n < 3000000) { p.vx_f = p.vx_a = 1; p.rows_f = 8; p.rows_a = 12; }
-  else if (n < 8000000) { p.vx_f = 2; p.vx_a = 1; p.rows_f = p.rows_a = 16; }
-  else if (n < 40000000) { p.vx_f = 4; p.vx_a = 2; p.rows_f = p.rows_a = 16; }
-  else { p.vx_f = p.vx_a = 4; p.rows_f = p.rows_a = 32; }
-  p.vx_f = std::min(p.vx_f, wide);
-  p.vx_a = std::min(p.vx_a, wide);
-  if (vec_x) p.vx_f = p.vx_a = vec_x;
-  if (rows) p.rows_f = p.rows_a = rows;
-  return p;
-}
 
 // Workspace (in floats): coefficient planes, two sets of receiver rows, the
 // receivers' cells (forward) or chains (adjoint).

@@ -97,7 +97,7 @@ template <int T, int VX, bool EDGE, bool RINGCOLS>
 __device__ __forceinline__ void el_march_strip(const ElParams& p, Const<ElParams> pc, int b,
                                                int strip, int seg) {
   constexpr int kAhead = 2;
-  const Lane l = make_lane<T, VX>(strip, p.g.nx);
+  const Lane l = make_lane<T, VX>(strip, p.sp, p.g.nx);
   const int64_t plane = p.g.plane, off = (int64_t)b * plane;
   const int nz = p.g.nz;
   const int z0 = seg * p.sp.rows, z1 = min(z0 + p.sp.rows, nz);  // owned rows

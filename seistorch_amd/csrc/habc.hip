@@ -23,10 +23,13 @@
 
 #include "common.h"
 #include "illum.h"
+#include "march.h"
+#include "march_rows.h"
 #include "seistorch_amd.h"
 #include "tiles.h"
 
 #include <initializer_list>
+#include <vector>
 
 using seis::Grid;
 using seis::lap_taps;
@@ -456,12 +459,13 @@ __device__ __forceinline__ int oneway_terms(int z, int x, int i, const float* __
 // With recon/grad (fused adjoint, y1 = lambda^{k+1}, y2 = lambda^{k+2}):
 // gradient 2c*A0*L(u^{k-1})*lambda^k on the interior (lambda^k without the
 // adjoint source, which k_habc_post adds with its gradient share) and the
-// interior rebuild of u^{k-2} over uc.  recon: 0 none, 1 rebuild, 2 zeros.
+// interior rebuild of u^{k-2} from u^k in uc into uo (the same buffer or
+// another).  recon: 0 none, 1 rebuild, 2 zeros.
 template <int S>
 __device__ __forceinline__ void habc_adj_cell(
     int z, int x, int grp, const float* __restrict__ vp, const float* __restrict__ bw,
     const float* __restrict__ y1, const float* __restrict__ y2, float* __restrict__ out,
-    const float* __restrict__ um, float* __restrict__ uc, float* __restrict__ gpart,
+    const float* __restrict__ um, const float* uc, float* uo, float* __restrict__ gpart,
     const int32_t* __restrict__ src, const float* __restrict__ wn, int recon, int B,
     const HabcCtx& hc, const seis::TimeConsts& k, int ng = 1) {
   const Grid& g = hc.g;
@@ -517,9 +521,9 @@ __device__ __forceinline__ void habc_adj_cell(
         if (recon == 1) {
           float un = uc[off + i];
           if (z == src[2 * bb] && x == src[2 * bb + 1]) un -= w;
-          uc[off + i] = ((k.two_idt2 * um[off + i] + (c * c) * Lu) - un / A0) / B0;
+          uo[off + i] = ((k.two_idt2 * um[off + i] + (c * c) * Lu) - un / A0) / B0;
         } else if (recon == 2) {
-          uc[off + i] = 0.0f;
+          uo[off + i] = 0.0f;
         }
       }
     }
@@ -539,7 +543,7 @@ template <int S, int VB, bool TOP>
 __device__ __forceinline__ void habc_adj_band(
     int z, int x0, int grp, int ng, const float* __restrict__ vp, const float* __restrict__ bw,
     const float* __restrict__ y1, const float* __restrict__ y2, float* __restrict__ out,
-    const float* __restrict__ um, float* __restrict__ uc, float* __restrict__ gpart,
+    const float* __restrict__ um, const float* uc, float* uo, float* __restrict__ gpart,
     const int32_t* __restrict__ src, const float* __restrict__ wn, int recon, int B,
     const HabcCtx& hc, const seis::TimeConsts& k) {
   const Grid& g = hc.g;
@@ -682,11 +686,11 @@ __device__ __forceinline__ void habc_adj_band(
         }
         if (recon != 0) {
           if (allin) {
-            vstore<VB>(uc + off + i0, un);
+            vstore<VB>(uo + off + i0, un);
           } else {
 #pragma unroll
             for (int e = 0; e < VB; ++e)
-              if (in[e]) uc[off + i0 + e] = un[e];
+              if (in[e]) uo[off + i0 + e] = un[e];
           }
         }
       }
@@ -712,7 +716,7 @@ template <int S, bool LEFT>
 __device__ __forceinline__ void habc_adj_side(
     int z, int x, int grp, int ng, const float* __restrict__ vp, const float* __restrict__ bw,
     const float* __restrict__ y1, const float* __restrict__ y2, float* __restrict__ out,
-    const float* __restrict__ um, float* __restrict__ uc, float* __restrict__ gpart,
+    const float* __restrict__ um, const float* uc, float* uo, float* __restrict__ gpart,
     const int32_t* __restrict__ src, const float* __restrict__ wn, int recon, int B,
     const HabcCtx& hc, const seis::TimeConsts& k) {
   const Grid& g = hc.g;
@@ -795,9 +799,9 @@ __device__ __forceinline__ void habc_adj_side(
         if (recon == 1) {
           float un = uc[off + i];
           if (z == src[2 * bb] && x == src[2 * bb + 1]) un -= w;
-          uc[off + i] = ((k.two_idt2 * um[off + i] + (c * c) * Lu) - un / A0) / B0;
+          uo[off + i] = ((k.two_idt2 * um[off + i] + (c * c) * Lu) - un / A0) / B0;
         } else if (recon == 2) {
-          uc[off + i] = 0.0f;
+          uo[off + i] = 0.0f;
         }
       }
     }
@@ -809,7 +813,7 @@ template <int S>
 __global__ __launch_bounds__(256) void k_habc_adj(
     const float* __restrict__ vp, const float* __restrict__ bw, const float* __restrict__ y1,
     const float* __restrict__ y2, float* __restrict__ out, const float* __restrict__ um,
-    float* __restrict__ uc, float* __restrict__ gpart, const int32_t* __restrict__ src,
+    float* uc, float* __restrict__ gpart, const int32_t* __restrict__ src,
     const float* __restrict__ wn, int recon, int B, HabcCtx hc, seis::TimeConsts k,
     TileMap tm) {
   int tx, tzi, grp;
@@ -818,7 +822,7 @@ __global__ __launch_bounds__(256) void k_habc_adj(
   const int x = tx * kLanes + (int)(threadIdx.x % kLanes);
   const int z = tzi * kRowsOfThreads + (int)(threadIdx.x / kLanes);
   if (x >= g.nx || z >= g.nz) return;
-  habc_adj_cell<S>(z, x, grp, vp, bw, y1, y2, out, um, uc, gpart, src, wn, recon, B, hc, k);
+  habc_adj_cell<S>(z, x, grp, vp, bw, y1, y2, out, um, uc, uc, gpart, src, wn, recon, B, hc, k);
 }
 
 // Variable-density adjoint (acoustic_rho_habc.py:31-57), exact transpose of
@@ -1204,7 +1208,7 @@ template <int S>
 __device__ __forceinline__ bool habc_adj_strip_block(
     int w, const float* __restrict__ vp, const float* __restrict__ bw,
     const float* __restrict__ y1, const float* __restrict__ y2, float* __restrict__ out, const float* __restrict__ um,
-    float* __restrict__ uc, float* __restrict__ gpart, const int32_t* __restrict__ src,
+    const float* uc, float* uo, float* __restrict__ gpart, const int32_t* __restrict__ src,
     const float* __restrict__ wn, int recon, int B, const HabcCtx& hc,
     const seis::TimeConsts& k, const Deep& dp, const Frame& f, int ngf, int G,
     const TileMap& tb, int ngb, const TileMap& ts) {
@@ -1215,7 +1219,7 @@ __device__ __forceinline__ bool habc_adj_strip_block(
   if (w < nf) {
     int zc, xc, gc;
     if (frame_cell(f, w, zc, xc, gc))
-      habc_adj_cell<S>(zc, xc, gc * ngf, vp, bw, y1, y2, out, um, uc, gpart, src, wn, recon, B,
+      habc_adj_cell<S>(zc, xc, gc * ngf, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn, recon, B,
                        hc, k, min(ngf, G - gc * ngf));
     return true;
   }
@@ -1229,10 +1233,10 @@ __device__ __forceinline__ bool habc_adj_strip_block(
     if (x0 >= dp.x1 || r >= ztop + (g.nz - dp.z1)) return true;
     const int grp = gb * ngb, ng = min(ngb, G - grp);
     if (r < ztop)
-      habc_adj_band<S, VB, true>(r, x0, grp, ng, vp, bw, y1, y2, out, um, uc, gpart, src, wn,
+      habc_adj_band<S, VB, true>(r, x0, grp, ng, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn,
                                  recon, B, hc, k);
     else
-      habc_adj_band<S, VB, false>(dp.z1 + (r - ztop), x0, grp, ng, vp, bw, y1, y2, out, um, uc,
+      habc_adj_band<S, VB, false>(dp.z1 + (r - ztop), x0, grp, ng, vp, bw, y1, y2, out, um, uc, uo,
                                   gpart, src, wn, recon, B, hc, k);
     return true;
   }
@@ -1247,10 +1251,10 @@ __device__ __forceinline__ bool habc_adj_strip_block(
     if (z >= dp.z1 || (tx == 0 ? x >= dp.x0 : x >= g.nx)) return true;
     const int grp = gb * ngb, ng = min(ngb, G - grp);
     if (tx == 0)
-      habc_adj_side<S, true>(z, x, grp, ng, vp, bw, y1, y2, out, um, uc, gpart, src, wn, recon,
+      habc_adj_side<S, true>(z, x, grp, ng, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn, recon,
                              B, hc, k);
     else
-      habc_adj_side<S, false>(z, x, grp, ng, vp, bw, y1, y2, out, um, uc, gpart, src, wn, recon,
+      habc_adj_side<S, false>(z, x, grp, ng, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn, recon,
                               B, hc, k);
     return true;
   }
@@ -1265,7 +1269,7 @@ template <int S, int VX, int RZ>
 __device__ __forceinline__ void habc_adj_deep_tile(
     int tx, int tzi, int grp, const float* __restrict__ vp, const float* __restrict__ bw,
     const float* __restrict__ y1, const float* __restrict__ y2, float* __restrict__ out, const float* __restrict__ um,
-    float* __restrict__ uc, float* __restrict__ gpart, const int32_t* __restrict__ src,
+    const float* uc, float* uo, float* __restrict__ gpart, const int32_t* __restrict__ src,
     const float* __restrict__ wn, int recon, int B, const HabcCtx& hc,
     const seis::TimeConsts& k, const Deep& dp) {
   const Grid& g = hc.g;
@@ -1354,7 +1358,7 @@ __device__ __forceinline__ void habc_adj_deep_tile(
             un[e] = 0.0f;
           }
         }
-        if (recon != 0) vstore<VX>(uc + off + i, un);
+        if (recon != 0) vstore<VX>(uo + off + i, un);
       }
     }
   }
@@ -1380,16 +1384,16 @@ template <int S, int VX>
 __global__ __launch_bounds__(256) void k_habc_adj_deep(
     const float* __restrict__ vp, const float* __restrict__ bw, const float* __restrict__ y1,
     const float* __restrict__ y2, float* __restrict__ out, const float* __restrict__ um,
-    float* __restrict__ uc, float* __restrict__ gpart, const int32_t* __restrict__ src,
+    const float* uc, float* uo, float* __restrict__ gpart, const int32_t* __restrict__ src,
     const float* __restrict__ wn, int recon, int B, HabcCtx hc, seis::TimeConsts k, Deep dp,
     TileMap tm, Frame f, int ngf, int G, TileMap tb, int ngb, TileMap ts) {
-  if (habc_adj_strip_block<S>((int)blockIdx.x, vp, bw, y1, y2, out, um, uc, gpart, src, wn,
+  if (habc_adj_strip_block<S>((int)blockIdx.x, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn,
                               recon, B, hc, k, dp, f, ngf, G, tb, ngb, ts))
     return;
   const int w = (int)blockIdx.x - (f.per + tb.per + ts.per) * kXcds;
   int tx, tzi, grp;
   if (!tile_of_w(tm, w, tx, tzi, grp)) return;
-  habc_adj_deep_tile<S, VX, kHabcRZ>(tx, tzi, grp, vp, bw, y1, y2, out, um, uc, gpart, src, wn,
+  habc_adj_deep_tile<S, VX, kHabcRZ>(tx, tzi, grp, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn,
                                      recon, B, hc, k, dp);
 }
 
@@ -1431,18 +1435,20 @@ __global__ __launch_bounds__(256) void k_habc_vjp_model(const float* __restrict_
 }
 
 // After k_habc_adj in the fused adjoint: adjoint source s^k at the receivers
-// (and its gradient share 2c*A0*L(u^{k-1})*s^k), ring restore of u^{k-2}.
+// (and its gradient share 2c*A0*L(u^{k-1})*s^k) but for those in `skip`, ring
+// restore of u^{k-2}.
 __global__ __launch_bounds__(256) void k_habc_post(
     const float* __restrict__ vp, const float* __restrict__ um, float* __restrict__ uc,
     float* __restrict__ lam, float* __restrict__ gpart, const int64_t* __restrict__ rec,
     const float* __restrict__ rgrad, int64_t R, const float* __restrict__ ring_slot,
-    int64_t ring_len, int recon, int B, int S, Grid g, seis::TimeConsts k) {
+    int64_t ring_len, int recon, int B, int S, Grid g, seis::TimeConsts k, Deep skip) {
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < R) {
     const int64_t f = rec[t];
     const int64_t b = f / g.plane;
     const int i = (int)(f - b * g.plane);
     const int z = i / g.nx, x = i - z * g.nx;
+    if (in_deep(z, x, skip)) return;
     const float sk = rgrad[t];
     atomicAdd(lam + f, sk);
     if (seis::interior(z, x, g)) {
@@ -1602,6 +1608,178 @@ TileMap side_tiles(const Grid& g, const Deep& dp, int groups) {
   return m;
 }
 
+// ---- four time steps per launch away from the boundary
+
+// Core: the cells at least kW + 3 + kMaxT from every edge.  Within kMaxT cells of
+// it the step is the undamped one, so the marching waves of march.h take up to
+// kMaxT steps of Core in one launch from the fields at its start alone.  The frame
+// around Core takes its steps one by one, step t of T also on the T - t outermost
+// cells of Core, which the frame's next steps read and the march leaves to itself.
+// (With one step per launch everywhere the fields cross HBM once per step, which
+// is what bounded it: 16 shots of 900 x 2500, 105 us forward, 261 adjoint per step
+// with the records and rings, now 70 and 167: 34 and 72 of them the march, most of the
+// rest the frame's steps, bound by their loads' latency and long set-up per cell.)
+constexpr int kCoreMargin = kW + 3 + kMaxT;
+
+inline Deep core_of(int64_t nz, int64_t nx) {
+  const int v = widest(nx);
+  return Deep{kCoreMargin, (int)nz - kCoreMargin, (kCoreMargin + v - 1) / v * v,
+              ((int)nx - kCoreMargin) / v * v};
+}
+
+inline Deep shrunk(const Deep& c, int e) { return Deep{c.z0 + e, c.z1 - e, c.x0 + e, c.x1 - e}; }
+
+// What a launch's adjoint sources reach of Core: a source in the frame kMaxT - 1
+// cells away is in Core's last level.
+inline Deep reach_of(const Deep& core) { return shrunk(core, 1 - kMaxT); }
+
+// Shot groups per thread of the frame's steps: a launch of its own needs enough
+// threads (about 400 thousand) before the set-up per cell is worth sharing.  us per
+// step, forward / adjoint, with groups of two shots: 300 x 500 x 8 1 group 10.7 / 38, 2
+// 11.6 / 41, 4 15.3 / 51; 900 x 2500 x 4 1 group 20.4 / 72, 2 20.0 / 68; x 16 1 group 75.6 /
+// 202, 2 70.1 / 179, 4 69.9 / 167, 8 72.5 / 177.
+inline int frame_groups(int64_t nz, int64_t nx, int G) {
+  const int64_t threads = 2 * kCoreMargin * (nz + nx) * G;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(4, (threads + 200000) / 400000));
+}
+
+// row_slot[z] = 0 for every row that holds a receiver in `in` (-1 before).
+__global__ __launch_bounds__(256) void k_core_rows(const int64_t* __restrict__ rec, int64_t R,
+                                                   int64_t plane, int nx, Deep in,
+                                                   int32_t* __restrict__ row_slot) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= R) return;
+  const int i = (int)(rec[t] % plane), z = i / nx;
+  if (in_deep(z, i - z * nx, in)) row_slot[z] = 0;
+}
+
+// Cells of the receivers in `part` in the (slots, B, nx) rows, -1 for the others; with
+// head/next, the receivers of one cell are chained for the adjoint's sources.
+__global__ __launch_bounds__(256) void k_core_cells(const int64_t* __restrict__ rec, int64_t R,
+                                                    int64_t plane, int nx, int B, Deep part,
+                                                    const int32_t* __restrict__ row_slot,
+                                                    int64_t* __restrict__ cell,
+                                                    int32_t* __restrict__ head,
+                                                    int32_t* __restrict__ next) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= R) return;
+  const int64_t b = rec[t] / plane;
+  const int i = (int)(rec[t] - b * plane), z = i / nx, x = i - z * nx;
+  const bool in = in_deep(z, x, part) && row_slot && row_slot[z] >= 0;
+  const int64_t c = in ? ((int64_t)row_slot[z] * B + b) * nx + x : -1;
+  if (cell) cell[t] = c;
+  if (head && in) next[t] = atomicExch(head + c, (int32_t)t);
+}
+
+struct CoreFwd {
+  FwdParams p;
+  int per;
+};
+
+struct CoreAdj {
+  AdjParams p;
+  int per;
+};
+
+template <int T, int VX>
+__global__ __launch_bounds__(kThreads) void k_core_fwd(CoreFwd a) {
+  int strip, seg, b;
+  if (!march_unit(a.p.sp, a.p.B, xcd_block(a.per), strip, seg, b)) return;
+  march_forward_strip<T, VX, false>(a.p, launch_params<FwdParams>(), b, strip, seg);
+}
+
+template <int T, int VX>
+__global__ __launch_bounds__(kThreads) void k_core_adj(CoreAdj a) {
+  int strip, seg, b;
+  if (!march_unit(a.p.sp, a.p.B, xcd_block(a.per), strip, seg, b)) return;
+  march_adjoint_strip<T, VX, kDeep>(a.p, launch_params<AdjParams>(), b, strip, seg);
+}
+
+#define SEIS_CORE_LAUNCH(K, T, VX, a, s)                                            \
+  switch (T * 8 + VX) {                                                             \
+    case 9: K<1, 1><<<a.per * kXcds, kThreads, 0, s>>>(a); break;                   \
+    case 10: K<1, 2><<<a.per * kXcds, kThreads, 0, s>>>(a); break;                  \
+    case 12: K<1, 4><<<a.per * kXcds, kThreads, 0, s>>>(a); break;                  \
+    case 17: K<2, 1><<<a.per * kXcds, kThreads, 0, s>>>(a); break;                  \
+    case 18: K<2, 2><<<a.per * kXcds, kThreads, 0, s>>>(a); break;                  \
+    case 20: K<2, 4><<<a.per * kXcds, kThreads, 0, s>>>(a); break;                  \
+    case 33: K<4, 1><<<a.per * kXcds, kThreads, 0, s>>>(a); break;                  \
+    case 34: K<4, 2><<<a.per * kXcds, kThreads, 0, s>>>(a); break;                  \
+    default: K<4, 4><<<a.per * kXcds, kThreads, 0, s>>>(a); break;                  \
+  }                                                                                 \
+  SEIS_CHECK_LAUNCH();
+
+// Records and rings of a launch's levels: receivers in Core from the rows, the
+// others and the rings from the levels' fields.
+struct CoreKeep {
+  const float* lev[kMaxT];
+  const float* rows;
+  const int64_t* cell;
+  const int64_t* rec;
+  int64_t R, row_cells, ring_len;
+  float* out;   // records of the first level
+  float* ring;  // ring slot of the first level
+  int ring_levels, B;
+};
+
+__global__ __launch_bounds__(256) void k_core_keep(CoreKeep a, Grid g) {
+  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int l = blockIdx.y;
+  const float* u = a.lev[l];
+  if (t < a.R) {
+    const int64_t c = a.cell[t];
+    a.out[l * a.R + t] = c >= 0 ? a.rows[l * a.row_cells + c] : u[a.rec[t]];
+    return;
+  }
+  t -= a.R;
+  if (l < a.ring_levels && t < (int64_t)a.B * a.ring_len) {
+    const int64_t b = t / a.ring_len;
+    const int64_t j = t - b * a.ring_len;
+    a.ring[l * a.B * a.ring_len + t] = u[b * g.plane + seis::ring_cell(j, g)];
+  }
+}
+
+// grad: on Core 2c A0 times the march's sums over the shots' planes, elsewhere the
+// frame's sums over the shot groups'.
+__global__ __launch_bounds__(256) void k_core_grad(const float* __restrict__ vp,
+                                                   const float* __restrict__ gcore, int nb,
+                                                   const float* __restrict__ gpart, int G,
+                                                   float* __restrict__ out, Deep core, Grid g,
+                                                   seis::TimeConsts k) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= g.plane) return;
+  const int z = (int)(t / g.nx), x = (int)(t - (int64_t)z * g.nx);
+  float s = 0.0f;
+  if (in_deep(z, x, core)) {
+    for (int b = 0; b < nb; ++b) s += gcore[b * g.plane + t];
+    s = 2.0f * vp[t] * (1.0f / k.idt2) * s;
+  } else {
+    for (int q = 0; q < G; ++q) s += gpart[(int64_t)q * g.plane + t];
+  }
+  out[t] = s;
+}
+
+struct CoreWork {
+  float *c2, *A, *Bc, *rows;
+  int64_t* cell;
+  int32_t *head, *next;
+  int64_t row_cells, total;
+};
+
+CoreWork carve_core(float* base, int64_t B, int64_t nz, int64_t nx, int64_t slots, int64_t R) {
+  CoreWork w;
+  int64_t o = 0;
+  auto take = [&](int64_t n) { const int64_t at = o; o += pad64(n); return base + at; };
+  w.row_cells = slots * B * nx;
+  w.c2 = take(nz * nx); w.A = take(nz * nx); w.Bc = take(nz * nx);
+  w.rows = take(kMaxT * w.row_cells);
+  w.cell = reinterpret_cast<int64_t*>(take(2 * R));
+  w.head = reinterpret_cast<int32_t*>(take(w.row_cells));
+  w.next = reinterpret_cast<int32_t*>(take(R));
+  w.total = o;
+  return w;
+}
+
 int habc_check(int64_t B, int64_t nz, int64_t nx, float dt, float h, int S) {
   SEIS_CHECK_ARG(B >= 1 && B <= 65535, "batch size %lld outside [1, 65535]", (long long)B);
   SEIS_CHECK_ARG(nz >= 2 * kW + 2 && nx >= 2 * kW + 2,
@@ -1610,6 +1788,21 @@ int habc_check(int64_t B, int64_t nz, int64_t nx, float dt, float h, int S) {
   SEIS_CHECK_ARG(nz * nx < (int64_t)1 << 31, "grid too large");
   SEIS_CHECK_ARG(dt > 0.0f && h > 0.0f, "dt and h must be positive");
   SEIS_CHECK_ARG(S == 1 || S == 2 || S == 4 || S == 8, "shots_per_group %d not in {1,2,4,8}", S);
+  return 0;
+}
+
+int check_core(int64_t nz, int64_t nx, int64_t R, int32_t slots, const int32_t* row_slot,
+               int32_t vec_x, int32_t rows) {
+  const Deep c = core_of(nz, nx);
+  SEIS_CHECK_ARG(nz * nx <= kMaxCells && c.z1 - c.z0 >= 4 * kMaxT && c.x1 - c.x0 >= 4 * kMaxT,
+                 "grid %lld x %lld has too few cells away from its edges", (long long)nz,
+                 (long long)nx);
+  SEIS_CHECK_ARG(slots >= 0 && slots <= nz && (slots == 0 || (row_slot && R > 0)) &&
+                     R < (int64_t)1 << 31,
+                 "receivers need their rows (slots %d)", slots);
+  SEIS_CHECK_ARG(vec_x == 0 || ((vec_x == 1 || vec_x == 2 || vec_x == 4) && nx % vec_x == 0),
+                 "vec_x %d for nx = %lld", vec_x, (long long)nx);
+  SEIS_CHECK_ARG(rows >= 0 && rows <= 1 << 20, "rows %d", rows);
   return 0;
 }
 
@@ -1959,7 +2152,7 @@ int seis_habc_backward(const float* vp, const float* b, const float* wavelet, in
     SEIS_PROF(SEIS_KERNEL_HABC_BWD, s);
     SEIS_HABC_LAUNCH_V(k_habc_adj_deep, S, VX,
                        dim3((tmd.per + fr.per + tmb.per + tms.per) * kXcds), s, vp, b, L1, L2,
-                       L0, X, Y, grad_part, src_zx, wavelet + (kk - 1), recon, (int)B, hc, k,
+                       L0, X, Y, Y, grad_part, src_zx, wavelet + (kk - 1), recon, (int)B, hc, k,
                        dp, tmd, fr, ngf, G, tmb, ngb, tms);
     SEIS_PROF(SEIS_KERNEL_HABC_BWD, s);
     const int64_t work = R + (recon ? B * ring_len : 0);
@@ -1967,7 +2160,7 @@ int seis_habc_backward(const float* vp, const float* b, const float* wavelet, in
       const float* slot = recon == 1 ? ring + (kk - 3) * B * ring_len : nullptr;
       k_habc_post<<<nblk(work), 256, 0, s>>>(vp, X, Y, L0, grad_part, rec_flat,
                                              R ? rec_grad + (kk - 1) * R : nullptr, R, slot,
-                                             ring_len, recon, (int)B, S, g, k);
+                                             ring_len, recon, (int)B, S, g, k, Deep{0, 0, 0, 0});
       SEIS_CHECK_LAUNCH();
     }
     const int64_t m = kk - 2;
@@ -1980,6 +2173,304 @@ int seis_habc_backward(const float* vp, const float* b, const float* wavelet, in
     t = L2; L2 = L1; L1 = L0; L0 = t;
   }
   k_habc_sum<<<nblk(g.plane), 256, 0, s>>>(grad_part, G, grad, g.plane);
+  SEIS_CHECK_LAUNCH();
+  return 0;
+}
+
+// Core needs a few cells beyond what a launch's frame steps take of it.
+int32_t seis_habc_march_fits(int64_t nz, int64_t nx) {
+  const Deep c = core_of(nz, nx);
+  return nz * nx <= kMaxCells && c.z1 - c.z0 >= 4 * kMaxT && c.x1 - c.x0 >= 4 * kMaxT;
+}
+
+int seis_habc_core_rows(const int64_t* rec_flat, int64_t R, int64_t nz, int64_t nx,
+                        int32_t* row_slot, void* stream) {
+  SEIS_CHECK_ARG(row_slot && (R == 0 || rec_flat) && R >= 0, "bad arguments");
+  SEIS_CHECK_ARG(nz >= 1 && nx >= 1 && nz * nx < (int64_t)1 << 31, "grid %lld x %lld",
+                 (long long)nz, (long long)nx);
+  hipStream_t s = (hipStream_t)stream;
+  k_fill_i32<<<blocks_of(nz), 256, 0, s>>>(row_slot, nz, -1);
+  SEIS_CHECK_LAUNCH();
+  if (R > 0) {
+    k_core_rows<<<blocks_of(R), 256, 0, s>>>(rec_flat, R, nz * nx, (int)nx,
+                                             reach_of(core_of(nz, nx)), row_slot);
+    SEIS_CHECK_LAUNCH();
+  }
+  k_number_rows<<<1, 64, 0, s>>>(row_slot, (int)nz);
+  SEIS_CHECK_LAUNCH();
+  return 0;
+}
+
+int64_t seis_habc_march_workspace(int64_t B, int64_t nz, int64_t nx, int32_t slots, int64_t R) {
+  return carve_core(nullptr, B, nz, nx, slots, R).total;
+}
+
+int seis_habc_march_forward(const float* vp, const float* b, const float* wavelet, int64_t nt,
+                            const int32_t* src_zx, const int64_t* rec_flat, int64_t R,
+                            const int32_t* row_slot, int32_t slots, float* rec_out, float* ring,
+                            float* snaps, int32_t snap_every, float* work, float* const* fields,
+                            int32_t* final_fields, int64_t B, int64_t nz, int64_t nx, float dt,
+                            float h, int32_t npml, int32_t multiple, int32_t shots_per_group,
+                            int32_t vec_x, int32_t rows, void* stream) {
+  if (int e = habc_check(B, nz, nx, dt, h, shots_per_group)) return e;
+  if (int e = check_core(nz, nx, R, slots, row_slot, vec_x, rows)) return e;
+  SEIS_CHECK_ARG(vp && b && wavelet && src_zx && work && fields && final_fields,
+                 "null pointer argument");
+  SEIS_CHECK_ARG(nt >= 1 && R >= 0 && (R == 0 || (rec_flat && rec_out)), "bad receiver arguments");
+  for (int i = 0; i < 5; ++i) SEIS_CHECK_ARG(fields[i], "null field buffer");
+  const int64_t ring_len = ring ? seis_ring_len(nz, nx, npml, multiple) : 0;
+  SEIS_CHECK_ARG(!ring || ring_len > 0, "grid has no interior inside npml=%d", npml);
+  SEIS_CHECK_ARG(!snaps || snap_every > 0, "snapshots need snap_every > 0");
+  const HabcCtx hc{seis::make_grid(nz, nx, npml, multiple != 0), multiple ? 1 : 0, dt, h};
+  const Grid& g = hc.g;
+  const int S = shots_per_group, G = (int)((B + S - 1) / S);
+  const int ngf = frame_groups(nz, nx, G);
+  const Deep core = core_of(nz, nx);
+  const Plan pl = make_plan(B * (core.z1 - core.z0) * (core.x1 - core.x0), widest(nx), 0, vec_x,
+                            rows);
+  const seis::TimeConsts k = seis::make_consts(dt, h);
+  const CoreWork w = carve_core(work, B, nz, nx, slots, R);
+  hipStream_t s = (hipStream_t)stream;
+  const int64_t field = B * g.plane;
+  k_coefs<<<blocks_of(g.plane), 256, 0, s>>>(vp, nullptr, g.plane, k, w.c2, w.A, w.Bc);
+  SEIS_CHECK_LAUNCH();
+  if (R > 0) {
+    k_core_cells<<<blocks_of(R), 256, 0, s>>>(rec_flat, R, g.plane, g.nx, (int)B, core,
+                                              slots ? row_slot : nullptr, w.cell, nullptr,
+                                              nullptr);
+    SEIS_CHECK_LAUNCH();
+  }
+  float *cur = fields[0], *prev = fields[1];
+  std::vector<float*> free_bufs{fields[2], fields[3], fields[4]};
+  auto take = [&]() { float* q = free_bufs.back(); free_bufs.pop_back(); return q; };
+  for (float* q : {cur, prev}) {
+    k_habc_fill<<<nblk(field), 256, 0, s>>>(q, field);
+    SEIS_CHECK_LAUNCH();
+  }
+  const int64_t last_snap = snaps ? seis_snapshot_count(nt, snap_every) * snap_every : 0;
+  for (int64_t n = 0; n < nt;) {
+    int64_t stop = nt, m = 0;
+    if (last_snap > 0 && n <= last_snap) {
+      m = std::max<int64_t>(1, (n - 1 + snap_every) / snap_every) * snap_every;
+      stop = m + 1;
+    }
+    const int T = next_steps(stop - n, kMaxT);
+    // fields of the levels: the frame's are whole only around Core, the march's
+    // (the last two) on Core; the second of four takes u^{n-1}'s place
+    float* lev[kMaxT + 2] = {prev, cur};  // lev[t + 1] = u^{n+t}
+    float* spare = nullptr;
+    if (T == 4) {
+      spare = take();
+      lev[2] = spare;
+      lev[3] = prev;
+    }
+    if (T >= 2) lev[T] = take();
+    lev[T + 1] = take();
+    CoreFwd a{};
+    a.p.cf = Coefs{w.c2, w.A, w.Bc};
+    a.p.f.u = cur; a.p.f.up = prev;
+    a.p.f.o1 = lev[T + 1];
+    a.p.f.o0 = T >= 2 ? lev[T] : nullptr;
+    a.p.f.w = wavelet + n;
+    a.p.f.rows = slots ? w.rows : nullptr;
+    a.p.f.row_slot = row_slot;
+    a.p.f.slots = slots;
+    a.p.src = src_zx;
+    a.p.B = (int)B;
+    a.p.sp = make_split(Region{core.z0, core.z1, core.x0, core.x1}, T, pl.vx_f, pl.rows_f,
+                        (int)std::min<int64_t>(B, kShotGroup));
+    a.p.g = g;
+    a.p.k = k;
+    a.per = (int)((split_blocks(a.p.sp, B) + kXcds - 1) / kXcds);
+    SEIS_PROF(SEIS_KERNEL_HABC_FWD, s);
+    SEIS_CORE_LAUNCH(k_core_fwd, T, pl.vx_f, a, s);
+    for (int t = 1; t <= T; ++t) {
+      const Deep dp = shrunk(core, T - t);
+      const Frame fr = make_frame(g, dp, (G + ngf - 1) / ngf);
+      SEIS_HABC_LAUNCH_V(k_habc_fwd_deep, S, 1, dim3(fr.per * kXcds), s, vp, lev[t], lev[t - 1],
+                         lev[t + 1], src_zx, wavelet + n + t - 1, (int)B, hc, k, dp,
+                         (TileMap{0, 0, 0, 0}), b, fr, ngf, G);
+    }
+    SEIS_PROF(SEIS_KERNEL_HABC_FWD, s);
+    CoreKeep kp{};
+    for (int t = 1; t <= T; ++t) kp.lev[t - 1] = lev[t + 1];
+    kp.rows = w.rows; kp.cell = w.cell; kp.rec = rec_flat;
+    kp.R = R; kp.row_cells = w.row_cells; kp.ring_len = ring_len;
+    kp.out = R ? rec_out + n * R : nullptr;
+    kp.ring_levels = ring ? (int)std::min<int64_t>(T, nt - 1 - n) : 0;
+    kp.ring = kp.ring_levels > 0 ? ring + n * B * ring_len : nullptr;
+    kp.B = (int)B;
+    const int64_t items = R + (kp.ring_levels > 0 ? B * ring_len : 0);
+    if (items > 0) {
+      k_core_keep<<<dim3(nblk(items), T), 256, 0, s>>>(kp, g);
+      SEIS_CHECK_LAUNCH();
+    }
+    if (spare) free_bufs.push_back(spare);
+    free_bufs.push_back(prev);
+    if (T >= 2) free_bufs.push_back(cur);
+    prev = T >= 2 ? lev[T] : cur;
+    cur = lev[T + 1];
+    n += T;
+    if (m > 0 && n == stop) {
+      float* sp = snaps + (m / snap_every - 1) * 2 * field;
+      k_habc_copy2<<<nblk(field), 256, 0, s>>>(prev, sp, cur, sp + field, field);
+      SEIS_CHECK_LAUNCH();
+    }
+  }
+  for (int i = 0; i < 5; ++i) {
+    if (fields[i] == cur) final_fields[0] = i;
+    if (fields[i] == prev) final_fields[1] = i;
+  }
+  return 0;
+}
+
+int seis_habc_march_backward(const float* vp, const float* b, const float* wavelet, int64_t nt,
+                             const int32_t* src_zx, const int64_t* rec_flat, int64_t R,
+                             const int32_t* row_slot, int32_t slots, const float* rec_grad,
+                             const float* ring, const float* snaps, int32_t snap_every,
+                             float* work, float* const* u, float* const* lam, float* grad_core,
+                             float* grad_part, float* grad, int64_t B, int64_t nz, int64_t nx,
+                             float dt, float h, int32_t npml, int32_t multiple,
+                             int32_t shots_per_group, int32_t vec_x, int32_t rows, void* stream) {
+  if (int e = habc_check(B, nz, nx, dt, h, shots_per_group)) return e;
+  if (int e = check_core(nz, nx, R, slots, row_slot, vec_x, rows)) return e;
+  SEIS_CHECK_ARG(vp && b && wavelet && src_zx && work && u && lam && grad_core && grad_part &&
+                     grad,
+                 "null pointer argument");
+  SEIS_CHECK_ARG(nt >= 1 && R >= 0 && (R == 0 || (rec_flat && rec_grad)),
+                 "bad receiver arguments");
+  for (int i = 0; i < 5; ++i) SEIS_CHECK_ARG(lam[i] && (i == 4 || u[i]), "null field buffer");
+  const int64_t ring_len = seis_ring_len(nz, nx, npml, multiple);
+  SEIS_CHECK_ARG(ring_len > 0, "grid has no interior inside npml=%d", npml);
+  SEIS_CHECK_ARG(ring || nt <= 2, "ring storage is required for nt > 2");
+  SEIS_CHECK_ARG(!snaps || snap_every > 0, "snapshots need snap_every > 0");
+  const HabcCtx hc{seis::make_grid(nz, nx, npml, multiple != 0), multiple ? 1 : 0, dt, h};
+  const Grid& g = hc.g;
+  const int S = shots_per_group, G = (int)((B + S - 1) / S);
+  const int ngf = frame_groups(nz, nx, G), ngb = ngf;
+  const Deep core = core_of(nz, nx);
+  const Plan pl = make_plan(B * (core.z1 - core.z0) * (core.x1 - core.x0), widest(nx), 0, vec_x,
+                            rows);
+  const seis::TimeConsts k = seis::make_consts(dt, h);
+  const CoreWork w = carve_core(work, B, nz, nx, slots, R);
+  hipStream_t s = (hipStream_t)stream;
+  const int64_t field = B * g.plane;
+  k_coefs<<<blocks_of(g.plane), 256, 0, s>>>(vp, nullptr, g.plane, k, w.c2, w.A, w.Bc);
+  SEIS_CHECK_LAUNCH();
+  if (slots > 0) {
+    k_fill_i32<<<blocks_of(w.row_cells), 256, 0, s>>>(w.head, w.row_cells, -1);
+    SEIS_CHECK_LAUNCH();
+    k_core_cells<<<blocks_of(R), 256, 0, s>>>(rec_flat, R, g.plane, g.nx, (int)B,
+                                              reach_of(core), row_slot, nullptr, w.head, w.next);
+    SEIS_CHECK_LAUNCH();
+  }
+  float *X = u[1], *Y = u[0];      // u^{k-1}, u^k
+  float *M1 = lam[0], *M2 = lam[1];  // lambda^{k+1}, lambda^{k+2}
+  std::vector<float*> ufree{u[2], u[3]}, lfree{lam[2], lam[3], lam[4]};
+  auto take = [](std::vector<float*>& v) { float* q = v.back(); v.pop_back(); return q; };
+  for (float* q : {M1, M2}) {
+    k_habc_fill<<<nblk(field), 256, 0, s>>>(q, field);
+    SEIS_CHECK_LAUNCH();
+  }
+  k_habc_fill<<<nblk((int64_t)G * g.plane), 256, 0, s>>>(grad_part, (int64_t)G * g.plane);
+  SEIS_CHECK_LAUNCH();
+  const int64_t last_snap = snaps ? seis_snapshot_count(nt, snap_every) * snap_every : 0;
+  bool first = true;
+  // iteration 1 adds nothing (u^0 = 0)
+  for (int64_t kk = nt; kk >= 2;) {
+    int64_t left = kk - 1, m = 0;
+    if (last_snap > 0 && kk >= snap_every + 2) {
+      m = std::min<int64_t>(last_snap, (kk - 2) / snap_every * snap_every);
+      left = kk - 2 - m + 1;
+    }
+    const int T = next_steps(left, kMaxT);
+    // L[t + 1] = lambda^{kk+1-t}, U[t + 1] = u^{kk-1-t}; the frame's first levels of
+    // four take the place of fields that the march has read
+    float* L[kMaxT + 2] = {M2, M1};
+    float* U[kMaxT + 2] = {Y, X};
+    float* spare = nullptr;
+    if (T == 4) {
+      spare = take(lfree);
+      L[2] = spare;
+      L[3] = M2;
+      U[2] = Y;
+      U[3] = X;
+    }
+    if (T >= 2) {
+      L[T] = take(lfree);
+      U[T] = take(ufree);
+    }
+    L[T + 1] = take(lfree);
+    U[T + 1] = take(ufree);
+    CoreAdj a{};
+    a.p.cf = Coefs{w.c2, w.A, w.Bc};
+    a.p.f.x = X; a.p.f.y = Y; a.p.f.m1 = M1; a.p.f.m2 = M2;
+    a.p.f.ox = U[T + 1];
+    a.p.f.om1 = L[T + 1];
+    a.p.f.oy = T >= 2 ? U[T] : nullptr;
+    a.p.f.om2 = T >= 2 ? L[T] : nullptr;
+    a.p.f.gpart = grad_core;
+    a.p.f.first = first;
+    a.p.f.w = wavelet + (kk - 1);
+    a.p.f.rows = slots ? w.rows : nullptr;
+    a.p.f.row_slot = row_slot;
+    a.p.f.slots = slots;
+    a.p.src = src_zx;
+    a.p.B = (int)B;
+    a.p.sp = make_split(Region{core.z0, core.z1, core.x0, core.x1}, T, pl.vx_a, pl.rows_a,
+                        (int)std::min<int64_t>(B, kShotGroup));
+    a.p.g = g;
+    a.p.k = k;
+    a.p.rebuild_last = true;
+    a.per = (int)((split_blocks(a.p.sp, B) + kXcds - 1) / kXcds);
+    if (slots > 0) {
+      const Sources so{w.rows, w.head, w.next, R, w.row_cells, rec_grad + (kk - 1) * R, T,
+                       aux_blocks(w.row_cells)};
+      k_sources<<<so.blocks, kThreads, 0, s>>>(so);
+      SEIS_CHECK_LAUNCH();
+    }
+    SEIS_PROF(SEIS_KERNEL_HABC_BWD, s);
+    SEIS_CORE_LAUNCH(k_core_adj, T, pl.vx_a, a, s);
+    first = false;
+    for (int t = 1; t <= T; ++t) {
+      const int64_t kt = kk - t + 1;
+      const int recon = kt >= 3 ? 1 : 2;
+      const Deep dp = shrunk(core, T - t);
+      const Frame fr = make_frame(g, dp, (G + ngf - 1) / ngf, true);
+      const TileMap tmb = band_tiles(g, dp, kBandVX, (G + ngb - 1) / ngb);
+      const TileMap tms = side_tiles(g, dp, (G + ngb - 1) / ngb);
+      SEIS_HABC_LAUNCH_V(k_habc_adj_deep, S, 1, dim3((fr.per + tmb.per + tms.per) * kXcds), s, vp,
+                         b, L[t], L[t - 1], L[t + 1], U[t], U[t - 1], U[t + 1], grad_part, src_zx,
+                         wavelet + (kt - 1), recon, (int)B, hc, k, dp, (TileMap{0, 0, 0, 0}), fr,
+                         ngf, G, tmb, ngb, tms);
+      const int64_t items = R + B * ring_len;
+      const float* slot = recon == 1 ? ring + (kt - 3) * B * ring_len : nullptr;
+      k_habc_post<<<nblk(items), 256, 0, s>>>(vp, U[t], U[t + 1], L[t + 1], grad_part, rec_flat,
+                                              R ? rec_grad + (kt - 1) * R : nullptr, R, slot,
+                                              ring_len, recon, (int)B, S, g, k, dp);
+      SEIS_CHECK_LAUNCH();
+    }
+    SEIS_PROF(SEIS_KERNEL_HABC_BWD, s);
+    if (spare) lfree.push_back(spare);
+    lfree.push_back(M2);
+    ufree.push_back(Y);
+    if (T >= 2) {
+      lfree.push_back(M1);
+      ufree.push_back(X);
+    }
+    M2 = T >= 2 ? L[T] : M1;
+    Y = T >= 2 ? U[T] : X;
+    M1 = L[T + 1];
+    X = U[T + 1];
+    kk -= T;
+    if (m > 0 && kk == m + 1) {  // (u^{k-1}, u^k) = (u^m, u^{m+1}) from storage
+      const float* sp = snaps + (m / snap_every - 1) * 2 * field;
+      k_habc_copy2<<<nblk(field), 256, 0, s>>>(sp, X, sp + field, Y, field);
+      SEIS_CHECK_LAUNCH();
+    }
+  }
+  k_core_grad<<<nblk(g.plane), 256, 0, s>>>(vp, grad_core, first ? 0 : (int)B, grad_part, G, grad,
+                                            core, g, k);
   SEIS_CHECK_LAUNCH();
   return 0;
 }

@@ -33,21 +33,34 @@ __host__ __device__ constexpr int out_cols(int T, int VX) {
   return (kWave - 2 * halo_lanes(T, VX)) * VX;
 }
 
-// Strips x segments x shots of one grid, the shots in groups:
+// The cells a launch writes: rows [z0, z1), columns [x0, x1), the columns multiples
+// of the lanes' width.
+struct Region {
+  int z0, z1, x0, x1;
+};
+
+// Strips x segments x shots of a region, the shots in groups:
 // unit = ((shot group * segs + seg) * strips + strip) * group + shot in group.
 struct Split {
   int strips, segs, rows;  // rows per segment
   int group;               // shots per group
+  Region reg;
 };
 
-inline Split make_split(const Grid& g, int T, int VX, int rows, int group) {
+inline Split make_split(const Region& r, int T, int VX, int rows, int group) {
   Split s;
-  s.strips = (g.nx + out_cols(T, VX) - 1) / out_cols(T, VX);
-  s.segs = (g.nz + rows - 1) / rows;
-  s.rows = (g.nz + s.segs - 1) / s.segs;
-  s.segs = (g.nz + s.rows - 1) / s.rows;
+  const int nz = r.z1 - r.z0;
+  s.strips = (r.x1 - r.x0 + out_cols(T, VX) - 1) / out_cols(T, VX);
+  s.segs = (nz + rows - 1) / rows;
+  s.rows = (nz + s.segs - 1) / s.segs;
+  s.segs = (nz + s.rows - 1) / s.rows;
   s.group = group;
+  s.reg = r;
   return s;
+}
+
+inline Split make_split(const Grid& g, int T, int VX, int rows, int group) {
+  return make_split(Region{0, g.nz, 0, g.nx}, T, VX, rows, group);
 }
 
 // The value of the lane to the left (lane 0: 0) / right (lane 63: 0).
@@ -119,13 +132,13 @@ struct Lane {
 };
 
 template <int T, int VX>
-__device__ __forceinline__ Lane make_lane(int strip, int nx) {
+__device__ __forceinline__ Lane make_lane(int strip, const Split& sp, int nx) {
   Lane l;
   constexpr int HL = halo_lanes(T, VX);
   const int lane = (int)(threadIdx.x & (kWave - 1));
-  l.x0 = strip * out_cols(T, VX) + (lane - HL) * VX;
+  l.x0 = sp.reg.x0 + strip * out_cols(T, VX) + (lane - HL) * VX;
   const bool xin = l.x0 >= 0 && l.x0 < nx;
-  l.inner = xin && lane >= HL && lane < kWave - HL;
+  l.inner = xin && lane >= HL && lane < kWave - HL && l.x0 < sp.reg.x1;
   l.in = xin ? (uint32_t)l.x0 * 4u : kLaneOut;
   l.out = l.inner ? l.in : kLaneOut;
   return l;
@@ -217,9 +230,9 @@ template <int T, int VX, bool RINGCOLS>
 __device__ __forceinline__ void march_forward_strip(const FwdParams& p, Const<FwdParams> pc, int b,
                                                     int strip, int seg) {
   constexpr int kAhead = rows_ahead(VX);
-  const Lane l = make_lane<T, VX>(strip, p.g.nx);
+  const Lane l = make_lane<T, VX>(strip, p.sp, p.g.nx);
   const int64_t plane = p.g.plane;
-  const int z0 = seg * p.sp.rows, z1 = min(z0 + p.sp.rows, p.g.nz);  // owned rows
+  const int z0 = p.sp.reg.z0 + seg * p.sp.rows, z1 = min(z0 + p.sp.rows, p.sp.reg.z1);  // owned
   const int zs = z0 - T;
   const int64_t off = (int64_t)b * plane;
   const Buf U = make_buf(p.f.u + off, plane), UP = make_buf(p.f.up + off, plane);
@@ -392,16 +405,20 @@ struct AdjParams {
 // Kinds of a strip's segment (its halo included): kFrame touches no interior
 // cell (mu only), kCore holds undamped interior cells only (A and B are
 // constants there and no ring cell is met), kMixed is everything else.
-enum Kind { kFrame, kMixed, kCore };
+// kDeep is kCore for adjoint fields without the factor A, which goes to the
+// Laplacian's weights instead (the sources are added as they are), as the HABC
+// adjoint forms them.
+enum Kind { kFrame, kMixed, kCore, kDeep };
 
 template <int T, int VX, int KIND>
 __device__ __forceinline__ void march_adjoint_strip(const AdjParams& p, Const<AdjParams> pc, int b,
                                                     int strip, int seg) {
-  constexpr bool HAS_U = KIND != kFrame, EDGE = KIND == kMixed, CORE = KIND == kCore;
+  constexpr bool HAS_U = KIND != kFrame, EDGE = KIND == kMixed;
+  constexpr bool DEEP = KIND == kDeep, CORE = KIND == kCore || DEEP;
   constexpr int kAhead = rows_ahead(VX);
-  const Lane l = make_lane<T, VX>(strip, p.g.nx);
+  const Lane l = make_lane<T, VX>(strip, p.sp, p.g.nx);
   const int64_t plane = p.g.plane;
-  const int z0 = seg * p.sp.rows, z1 = min(z0 + p.sp.rows, p.g.nz);
+  const int z0 = p.sp.reg.z0 + seg * p.sp.rows, z1 = min(z0 + p.sp.rows, p.sp.reg.z1);
   const int zs = z0 - T;
   const int64_t off = (int64_t)b * plane;
   const Buf M1 = make_buf(p.f.m1 + off, plane), M2 = make_buf(p.f.m2 + off, plane);
@@ -417,6 +434,7 @@ __device__ __forceinline__ void march_adjoint_strip(const AdjParams& p, Const<Ad
   const float ih2 = p.k.ih2, two_idt2 = p.k.two_idt2;
   const float kA = 1.0f / p.k.idt2, kB = p.k.idt2;  // undamped A and B, as the forward forms them
   const float rA = 1.0f / kA, rB = 1.0f / kB;
+  const float ka = two_idt2 * kA, kb = -(kB * kA);  // DEEP
   const int sz = scalar_at(p.src, 2 * b);
   const int32_t* row_slot = p.f.rows ? p.f.row_slot : nullptr;
   // rows whose u is read; owned rows whose u is written; owned rows of the
@@ -550,7 +568,7 @@ __device__ __forceinline__ void march_adjoint_strip(const AdjParams& p, Const<Ad
         c2[(q + 3) & 3][e] = cC[e];
         cC[e] = nc2[q % kAhead][e];
         M[0][q][e] = nM1[q % kAhead][e];
-        Q[0][q][e] = cC[e] * M[0][q][e];
+        Q[0][q][e] = (DEEP ? cC[e] * kA : cC[e]) * M[0][q][e];
         PM[e] = nM2[q % kAhead][e];
         if constexpr (!CORE) {
           A[(q + 3) & 3][e] = nA[q % kAhead][e];
@@ -591,8 +609,11 @@ __device__ __forceinline__ void march_adjoint_strip(const AdjParams& p, Const<Ad
             float prev;
             if (t == 1) prev = PM[e];
             else prev = M[t >= 2 ? t - 2 : 0][(q - t) & 3][e];
-            V[e] = A[(q - t) & 3][e] *
-                   ((two_idt2 * M[t - 1][(q - t) & 3][e] - Bc[(q - t) & 3][e] * prev) + Lm);
+            if constexpr (DEEP)
+              V[e] = (ka * M[t - 1][(q - t) & 3][e] + Lm) + kb * prev;
+            else
+              V[e] = A[(q - t) & 3][e] *
+                     ((two_idt2 * M[t - 1][(q - t) & 3][e] - Bc[(q - t) & 3][e] * prev) + Lm);
           }
         }
         if (__builtin_expect((here >> (t - 1)) & 1u, 0)) {
@@ -601,13 +622,14 @@ __device__ __forceinline__ void march_adjoint_strip(const AdjParams& p, Const<Ad
           for (int e = 0; e < VX; ++e) s[e] = SR[e];
           if (t != t0) source_row(t, z, s);  // receivers on neighbouring rows
 #pragma unroll
-          for (int e = 0; e < VX; ++e) V[e] = V[e] + A[(q - t) & 3][e] * s[e];
+          for (int e = 0; e < VX; ++e)
+            V[e] = V[e] + (DEEP ? s[e] : A[(q - t) & 3][e] * s[e]);
         }
         if (t < T) {
 #pragma unroll
           for (int e = 0; e < VX; ++e) {
             M[t < T ? t : 0][(q - t) & 3][e] = V[e];
-            Q[t < T ? t : 0][(q - t) & 3][e] = ca[e] * V[e];
+            Q[t < T ? t : 0][(q - t) & 3][e] = (DEEP ? ca[e] * kA : ca[e]) * V[e];
           }
         }
         if (t >= T - 1) {

@@ -19,8 +19,8 @@ interior reverses exactly as in the PML case).
 import torch
 
 from .. import _lib, library
-from .acoustic import (NPML, _check_acquisition, _f, check_finite, default_shots_per_group,
-                       restore_boundaries, step as _undamped_step)
+from .acoustic import (MARCH_ROW_SHARE, MARCH_ROWS, NPML, _check_acquisition, _f, check_finite,
+                       default_shots_per_group, restore_boundaries, step as _undamped_step)
 
 
 def _multiple(habcs):
@@ -62,6 +62,69 @@ def _time_step_backward_multiple(*args, **kwargs):
 
 # ----------------------------------------------------------------- fused loop
 
+def _march_fits(B, nz, nx):
+    """Whether the marching loops take the grid and pay for their launches of the
+    frame's steps.  us per step, forward / adjoint, one step per launch and
+    marching: 164 x 164 x 1 shot 6.4 / 24 and 6.5 / 26, 300 x 500 x 2 8.0 / 31 and
+    8.1 / 33, 900 x 2500 x 1 10.7 / 38 and 11.7 / 38, 300 x 500 x 8 15 / 50 and 10.7 /
+    38, 451 x 877 x 4 11.6 / 41 and 10.8 / 39, 900 x 2500 x 4 22 / 65 and 20 / 67, x
+    16 105 / 261 and 70 / 167."""
+    return B >= 4 and B * nz * nx >= 1000000 and bool(_lib.load().seis_habc_march_fits(nz, nx))
+
+
+def _march_rows(rec_flat, nz, nx):
+    """(row_slot int32 (nz + 1), count): the grid rows with receivers in the part
+    that the marching loops take, or None when there are too many."""
+    row_slot = torch.empty(nz + 1, dtype=torch.int32, device=rec_flat.device)
+    _lib.call("seis_habc_core_rows", _lib.ptr(rec_flat), rec_flat.shape[0], nz, nx,
+              _lib.ptr(row_slot), _lib.stream_of(rec_flat))
+    slots = int(row_slot[nz])
+    return (row_slot, slots) if slots <= max(MARCH_ROWS, nz // MARCH_ROW_SHARE) else None
+
+
+def _march_buffers(vp, rows, R, B, n_fields):
+    """n_fields (B, nz, nx) buffers and the workspace of a marching loop, or None
+    when they do not fit (the one-step loops need fewer)."""
+    nz, nx = vp.shape
+    n = int(_lib.load().seis_habc_march_workspace(B, nz, nx, rows[1], R))
+    try:
+        bufs = [torch.empty((B, nz, nx), device=vp.device) for _ in range(n_fields)]
+        return bufs, torch.empty(n, device=vp.device)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
+def _march_forward(bufs, work, vp, b, wavelet, src_zx, rec_flat, rows, rec, ring, snaps, K, B, dt,
+                   h, multiple, S, shape=(0, 0)):
+    """The loop with up to four time steps per launch -> (u^nt, u^{nt-1}).
+    shape: (cells per lane, rows per wave), 0 automatic."""
+    nz, nx = vp.shape
+    last = torch.zeros(2, dtype=torch.int32)
+    _lib.call("seis_habc_march_forward", _lib.ptr(vp), _lib.ptr(b), _lib.ptr(wavelet),
+              wavelet.shape[0], _lib.ptr(src_zx), _lib.ptr(rec_flat), rec_flat.shape[0],
+              _lib.ptr(rows[0]), rows[1], _lib.ptr(rec), _lib.ptr(ring), _lib.ptr(snaps),
+              K if snaps is not None else 0, _lib.ptr(work), _lib.ptr_array(bufs),
+              _lib.ptr(last), B, nz, nx, dt, h, NPML, int(multiple), S, *shape,
+              _lib.stream_of(vp))
+    return bufs[int(last[0])], bufs[int(last[1])]
+
+
+def _march_backward(bufs, work, vp, b, wavelet, src_zx, rec_flat, rows, grad_rec, ring, snaps, K,
+                    u_a, u_b, gpart, B, dt, h, multiple, S, shape=(0, 0)):
+    """The gradient with up to four reverse steps per launch; bufs: two more
+    forward fields, five adjoint fields and the shots' gradients."""
+    nz, nx = vp.shape
+    grad = torch.empty_like(vp)
+    _lib.call("seis_habc_march_backward", _lib.ptr(vp), _lib.ptr(b), _lib.ptr(wavelet),
+              wavelet.shape[0], _lib.ptr(src_zx), _lib.ptr(rec_flat), rec_flat.shape[0],
+              _lib.ptr(rows[0]), rows[1], _lib.ptr(grad_rec), _lib.ptr(ring), _lib.ptr(snaps),
+              K if snaps is not None else 0, _lib.ptr(work),
+              _lib.ptr_array([u_a, u_b, bufs[0], bufs[1]]), _lib.ptr_array(bufs[2:7]),
+              _lib.ptr(bufs[7]), _lib.ptr(gpart), _lib.ptr(grad), B, nz, nx, dt, h, NPML,
+              int(multiple), S, *shape, _lib.stream_of(vp))
+    return grad
+
+
 class HabcLoop(torch.autograd.Function):
     @staticmethod
     def forward(ctx, vp, b, wavelet, src_zx, rec_flat, B, dt, h, multiple, shots_per_group,
@@ -76,12 +139,18 @@ class HabcLoop(torch.autograd.Function):
         nz, nx = vp.shape
         nt = wavelet.shape[0]
         R = rec_flat.shape[0]
+        # up to four steps per launch away from the edges; a launch shape and the
+        # illumination keep one
+        rows = None
+        if shots_per_group is None and illum is None and _march_fits(B, nz, nx):
+            rows = _march_rows(rec_flat, nz, nx)
         if shots_per_group is None:
             from .. import autotune
             tuned = autotune.lookup("habc", B, nz, nx)
             shots_per_group = tuned[0] if tuned else None
-        S = int(shots_per_group or default_shots_per_group(B))
-        u = [torch.empty((B, nz, nx), device=vp.device) for _ in range(3)]
+        bufs = _march_buffers(vp, rows, R, B, 5) if rows else None
+        # the marching loops' frame steps in pairs of shots
+        S = min(B, 2) if bufs else int(shots_per_group or default_shots_per_group(B))
         rec = torch.empty((nt, R), device=vp.device)
         ring = snaps = None
         K = 0
@@ -94,14 +163,21 @@ class HabcLoop(torch.autograd.Function):
             n_snap = int(_lib.load().seis_snapshot_count(nt, K))
             if n_snap > 0:
                 snaps = torch.empty((n_snap, 2, B, nz, nx), device=vp.device)
-        _lib.call("seis_habc_forward", _lib.ptr(vp), _lib.ptr(b), _lib.ptr(wavelet), nt,
-                  _lib.ptr(src_zx), _lib.ptr(rec_flat), R, _lib.ptr(rec), _lib.ptr(ring),
-                  _lib.ptr(snaps), K, _lib.ptr(illum), _lib.ptr(u[0]), _lib.ptr(u[1]),
-                  _lib.ptr(u[2]), B, nz, nx, dt, h, NPML, int(multiple), S, _lib.stream_of(vp))
+        if bufs is not None:
+            u = _march_forward(*bufs, vp, b, wavelet, src_zx, rec_flat, rows, rec, ring, snaps, K,
+                               B, dt, h, multiple, S)
+            bufs = None
+        else:
+            u = [torch.empty((B, nz, nx), device=vp.device) for _ in range(3)]
+            _lib.call("seis_habc_forward", _lib.ptr(vp), _lib.ptr(b), _lib.ptr(wavelet), nt,
+                      _lib.ptr(src_zx), _lib.ptr(rec_flat), R, _lib.ptr(rec), _lib.ptr(ring),
+                      _lib.ptr(snaps), K, _lib.ptr(illum), _lib.ptr(u[0]), _lib.ptr(u[1]),
+                      _lib.ptr(u[2]), B, nz, nx, dt, h, NPML, int(multiple), S,
+                      _lib.stream_of(vp))
         check_finite(rec)
         if need_grad:
             ctx.save_for_backward(vp, b, wavelet, src_zx, rec_flat)
-            ctx.state = (ring, snaps, u[0], u[1])
+            ctx.state = (ring, snaps, u[0], u[1], rows)
             ctx.meta = (B, dt, h, S, K, int(multiple))
         return rec
 
@@ -109,19 +185,25 @@ class HabcLoop(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, grad_rec):
         vp, b, wavelet, src_zx, rec_flat = ctx.saved_tensors
-        ring, snaps, u_a, u_b = ctx.state
+        ring, snaps, u_a, u_b, rows = ctx.state
         ctx.state = None
         B, dt, h, S, K, multiple = ctx.meta
         nz, nx = vp.shape
         nt = wavelet.shape[0]
         R = rec_flat.shape[0]
         G = (B + S - 1) // S
-        lam = [torch.empty_like(u_a) for _ in range(3)]
+        grad_rec = grad_rec.contiguous().float()
         gpart = torch.empty((G, nz, nx), device=vp.device)
+        bufs = _march_buffers(vp, rows, R, B, 8) if rows else None
+        if bufs is not None:
+            grad = _march_backward(*bufs, vp, b, wavelet, src_zx, rec_flat, rows, grad_rec, ring,
+                                   snaps, K, u_a, u_b, gpart, B, dt, h, multiple, S)
+            return (grad,) + (None,) * 11
+        lam = [torch.empty_like(u_a) for _ in range(3)]
         grad = torch.empty_like(vp)
         _lib.call("seis_habc_backward", _lib.ptr(vp), _lib.ptr(b), _lib.ptr(wavelet), nt,
                   _lib.ptr(src_zx), _lib.ptr(rec_flat), R,
-                  _lib.ptr(grad_rec.contiguous().float()), _lib.ptr(ring), _lib.ptr(snaps),
+                  _lib.ptr(grad_rec), _lib.ptr(ring), _lib.ptr(snaps),
                   K if snaps is not None else 0, _lib.ptr(u_a), _lib.ptr(u_b), _lib.ptr(lam[0]),
                   _lib.ptr(lam[1]), _lib.ptr(lam[2]), _lib.ptr(gpart), _lib.ptr(grad), B, nz, nx,
                   dt, h, NPML, multiple, S, _lib.stream_of(vp))
