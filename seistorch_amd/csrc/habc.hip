@@ -459,13 +459,13 @@ __device__ __forceinline__ int oneway_terms(int z, int x, int i, const float* __
 // With recon/grad (fused adjoint, y1 = lambda^{k+1}, y2 = lambda^{k+2}):
 // gradient 2c*A0*L(u^{k-1})*lambda^k on the interior (lambda^k without the
 // adjoint source, which k_habc_post adds with its gradient share) and the
-// interior rebuild of u^{k-2} from u^k in uc into uo (the same buffer or
-// another).  recon: 0 none, 1 rebuild, 2 zeros.
-template <int S>
+// interior rebuild of u^{k-2} from u^k in uc over uc (SAME) or
+// into uo.  recon: 0 none, 1 rebuild, 2 zeros.
+template <int S, bool SAME>
 __device__ __forceinline__ void habc_adj_cell(
     int z, int x, int grp, const float* __restrict__ vp, const float* __restrict__ bw,
     const float* __restrict__ y1, const float* __restrict__ y2, float* __restrict__ out,
-    const float* __restrict__ um, const float* uc, float* uo, float* __restrict__ gpart,
+    const float* __restrict__ um, float* __restrict__ uc, float* __restrict__ uo, float* __restrict__ gpart,
     const int32_t* __restrict__ src, const float* __restrict__ wn, int recon, int B,
     const HabcCtx& hc, const seis::TimeConsts& k, int ng = 1) {
   const Grid& g = hc.g;
@@ -521,9 +521,9 @@ __device__ __forceinline__ void habc_adj_cell(
         if (recon == 1) {
           float un = uc[off + i];
           if (z == src[2 * bb] && x == src[2 * bb + 1]) un -= w;
-          uo[off + i] = ((k.two_idt2 * um[off + i] + (c * c) * Lu) - un / A0) / B0;
+          (SAME ? uc : uo)[off + i] = ((k.two_idt2 * um[off + i] + (c * c) * Lu) - un / A0) / B0;
         } else if (recon == 2) {
-          uo[off + i] = 0.0f;
+          (SAME ? uc : uo)[off + i] = 0.0f;
         }
       }
     }
@@ -539,11 +539,11 @@ __device__ __forceinline__ void habc_adj_cell(
 // So a lane takes VB consecutive cells of one row, every access is a row
 // vector, and each cell sums the same operands in the same order as
 // habc_adj_cell (bit-identical).  TOP: the top band, else the bottom band.
-template <int S, int VB, bool TOP>
+template <int S, int VB, bool TOP, bool SAME>
 __device__ __forceinline__ void habc_adj_band(
     int z, int x0, int grp, int ng, const float* __restrict__ vp, const float* __restrict__ bw,
     const float* __restrict__ y1, const float* __restrict__ y2, float* __restrict__ out,
-    const float* __restrict__ um, const float* uc, float* uo, float* __restrict__ gpart,
+    const float* __restrict__ um, float* __restrict__ uc, float* __restrict__ uo, float* __restrict__ gpart,
     const int32_t* __restrict__ src, const float* __restrict__ wn, int recon, int B,
     const HabcCtx& hc, const seis::TimeConsts& k) {
   const Grid& g = hc.g;
@@ -686,11 +686,11 @@ __device__ __forceinline__ void habc_adj_band(
         }
         if (recon != 0) {
           if (allin) {
-            vstore<VB>(uo + off + i0, un);
+            vstore<VB>((SAME ? uc : uo) + off + i0, un);
           } else {
 #pragma unroll
             for (int e = 0; e < VB; ++e)
-              if (in[e]) uo[off + i0 + e] = un[e];
+              if (in[e]) (SAME ? uc : uo)[off + i0 + e] = un[e];
           }
         }
       }
@@ -712,11 +712,11 @@ __device__ __forceinline__ void habc_adj_band(
 // which terms exist depends on the column alone.  Same operands in the same
 // order as habc_adj_cell (bit-identical).  LEFT: the left column, else the
 // right one.
-template <int S, bool LEFT>
+template <int S, bool LEFT, bool SAME>
 __device__ __forceinline__ void habc_adj_side(
     int z, int x, int grp, int ng, const float* __restrict__ vp, const float* __restrict__ bw,
     const float* __restrict__ y1, const float* __restrict__ y2, float* __restrict__ out,
-    const float* __restrict__ um, const float* uc, float* uo, float* __restrict__ gpart,
+    const float* __restrict__ um, float* __restrict__ uc, float* __restrict__ uo, float* __restrict__ gpart,
     const int32_t* __restrict__ src, const float* __restrict__ wn, int recon, int B,
     const HabcCtx& hc, const seis::TimeConsts& k) {
   const Grid& g = hc.g;
@@ -799,9 +799,9 @@ __device__ __forceinline__ void habc_adj_side(
         if (recon == 1) {
           float un = uc[off + i];
           if (z == src[2 * bb] && x == src[2 * bb + 1]) un -= w;
-          uo[off + i] = ((k.two_idt2 * um[off + i] + (c * c) * Lu) - un / A0) / B0;
+          (SAME ? uc : uo)[off + i] = ((k.two_idt2 * um[off + i] + (c * c) * Lu) - un / A0) / B0;
         } else if (recon == 2) {
-          uo[off + i] = 0.0f;
+          (SAME ? uc : uo)[off + i] = 0.0f;
         }
       }
     }
@@ -822,7 +822,7 @@ __global__ __launch_bounds__(256) void k_habc_adj(
   const int x = tx * kLanes + (int)(threadIdx.x % kLanes);
   const int z = tzi * kRowsOfThreads + (int)(threadIdx.x / kLanes);
   if (x >= g.nx || z >= g.nz) return;
-  habc_adj_cell<S>(z, x, grp, vp, bw, y1, y2, out, um, uc, uc, gpart, src, wn, recon, B, hc, k);
+  habc_adj_cell<S, true>(z, x, grp, vp, bw, y1, y2, out, um, uc, nullptr, gpart, src, wn, recon, B, hc, k);
 }
 
 // Variable-density adjoint (acoustic_rho_habc.py:31-57), exact transpose of
@@ -1204,11 +1204,11 @@ __global__ __launch_bounds__(256) void k_rho_adj_grad(
 // per ngf groups); the next tb.per*8 the top and bottom bands in lane vectors
 // for ngb groups; the next ts.per*8 the left and right columns over Deep's
 // rows, one cell per lane for ngb groups.
-template <int S>
+template <int S, bool SAME>
 __device__ __forceinline__ bool habc_adj_strip_block(
     int w, const float* __restrict__ vp, const float* __restrict__ bw,
     const float* __restrict__ y1, const float* __restrict__ y2, float* __restrict__ out, const float* __restrict__ um,
-    const float* uc, float* uo, float* __restrict__ gpart, const int32_t* __restrict__ src,
+    float* __restrict__ uc, float* __restrict__ uo, float* __restrict__ gpart, const int32_t* __restrict__ src,
     const float* __restrict__ wn, int recon, int B, const HabcCtx& hc,
     const seis::TimeConsts& k, const Deep& dp, const Frame& f, int ngf, int G,
     const TileMap& tb, int ngb, const TileMap& ts) {
@@ -1219,7 +1219,7 @@ __device__ __forceinline__ bool habc_adj_strip_block(
   if (w < nf) {
     int zc, xc, gc;
     if (frame_cell(f, w, zc, xc, gc))
-      habc_adj_cell<S>(zc, xc, gc * ngf, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn, recon, B,
+      habc_adj_cell<S, SAME>(zc, xc, gc * ngf, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn, recon, B,
                        hc, k, min(ngf, G - gc * ngf));
     return true;
   }
@@ -1233,10 +1233,10 @@ __device__ __forceinline__ bool habc_adj_strip_block(
     if (x0 >= dp.x1 || r >= ztop + (g.nz - dp.z1)) return true;
     const int grp = gb * ngb, ng = min(ngb, G - grp);
     if (r < ztop)
-      habc_adj_band<S, VB, true>(r, x0, grp, ng, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn,
+      habc_adj_band<S, VB, true, SAME>(r, x0, grp, ng, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn,
                                  recon, B, hc, k);
     else
-      habc_adj_band<S, VB, false>(dp.z1 + (r - ztop), x0, grp, ng, vp, bw, y1, y2, out, um, uc, uo,
+      habc_adj_band<S, VB, false, SAME>(dp.z1 + (r - ztop), x0, grp, ng, vp, bw, y1, y2, out, um, uc, uo,
                                   gpart, src, wn, recon, B, hc, k);
     return true;
   }
@@ -1251,10 +1251,10 @@ __device__ __forceinline__ bool habc_adj_strip_block(
     if (z >= dp.z1 || (tx == 0 ? x >= dp.x0 : x >= g.nx)) return true;
     const int grp = gb * ngb, ng = min(ngb, G - grp);
     if (tx == 0)
-      habc_adj_side<S, true>(z, x, grp, ng, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn, recon,
+      habc_adj_side<S, true, SAME>(z, x, grp, ng, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn, recon,
                              B, hc, k);
     else
-      habc_adj_side<S, false>(z, x, grp, ng, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn, recon,
+      habc_adj_side<S, false, SAME>(z, x, grp, ng, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn, recon,
                               B, hc, k);
     return true;
   }
@@ -1265,11 +1265,11 @@ __device__ __forceinline__ bool habc_adj_strip_block(
 // every edge, x0 and x1 multiples of VX): there no strip term reaches, so a
 // lane runs a vectorised copy of the per-cell deep path of habc_adj_cell with
 // the same operands in the same order (bit-identical), for RZ rows.
-template <int S, int VX, int RZ>
+template <int S, int VX, int RZ, bool SAME>
 __device__ __forceinline__ void habc_adj_deep_tile(
     int tx, int tzi, int grp, const float* __restrict__ vp, const float* __restrict__ bw,
     const float* __restrict__ y1, const float* __restrict__ y2, float* __restrict__ out, const float* __restrict__ um,
-    const float* uc, float* uo, float* __restrict__ gpart, const int32_t* __restrict__ src,
+    float* __restrict__ uc, float* __restrict__ uo, float* __restrict__ gpart, const int32_t* __restrict__ src,
     const float* __restrict__ wn, int recon, int B, const HabcCtx& hc,
     const seis::TimeConsts& k, const Deep& dp) {
   const Grid& g = hc.g;
@@ -1358,7 +1358,7 @@ __device__ __forceinline__ void habc_adj_deep_tile(
             un[e] = 0.0f;
           }
         }
-        if (recon != 0) vstore<VX>(uo + off + i, un);
+        if (recon != 0) vstore<VX>((SAME ? uc : uo) + off + i, un);
       }
     }
   }
@@ -1380,20 +1380,20 @@ __device__ __forceinline__ void habc_adj_deep_tile(
 // vectors (one row per thread: the kernel's register count, and so the strip
 // threads' occupancy, follows the larger branch).  Requires y1, y2, um and
 // gpart (the fused loop's call).
-template <int S, int VX>
+template <int S, int VX, bool SAME>
 __global__ __launch_bounds__(256) void k_habc_adj_deep(
     const float* __restrict__ vp, const float* __restrict__ bw, const float* __restrict__ y1,
     const float* __restrict__ y2, float* __restrict__ out, const float* __restrict__ um,
-    const float* uc, float* uo, float* __restrict__ gpart, const int32_t* __restrict__ src,
+    float* __restrict__ uc, float* __restrict__ uo, float* __restrict__ gpart, const int32_t* __restrict__ src,
     const float* __restrict__ wn, int recon, int B, HabcCtx hc, seis::TimeConsts k, Deep dp,
     TileMap tm, Frame f, int ngf, int G, TileMap tb, int ngb, TileMap ts) {
-  if (habc_adj_strip_block<S>((int)blockIdx.x, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn,
+  if (habc_adj_strip_block<S, SAME>((int)blockIdx.x, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn,
                               recon, B, hc, k, dp, f, ngf, G, tb, ngb, ts))
     return;
   const int w = (int)blockIdx.x - (f.per + tb.per + ts.per) * kXcds;
   int tx, tzi, grp;
   if (!tile_of_w(tm, w, tx, tzi, grp)) return;
-  habc_adj_deep_tile<S, VX, kHabcRZ>(tx, tzi, grp, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn,
+  habc_adj_deep_tile<S, VX, kHabcRZ, SAME>(tx, tzi, grp, vp, bw, y1, y2, out, um, uc, uo, gpart, src, wn,
                                      recon, B, hc, k, dp);
 }
 
@@ -1437,6 +1437,7 @@ __global__ __launch_bounds__(256) void k_habc_vjp_model(const float* __restrict_
 // After k_habc_adj in the fused adjoint: adjoint source s^k at the receivers
 // (and its gradient share 2c*A0*L(u^{k-1})*s^k) but for those in `skip`, ring
 // restore of u^{k-2}.
+template <bool SKIP>
 __global__ __launch_bounds__(256) void k_habc_post(
     const float* __restrict__ vp, const float* __restrict__ um, float* __restrict__ uc,
     float* __restrict__ lam, float* __restrict__ gpart, const int64_t* __restrict__ rec,
@@ -1445,11 +1446,11 @@ __global__ __launch_bounds__(256) void k_habc_post(
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < R) {
     const int64_t f = rec[t];
+    const float sk = rgrad[t];
     const int64_t b = f / g.plane;
     const int i = (int)(f - b * g.plane);
     const int z = i / g.nx, x = i - z * g.nx;
-    if (in_deep(z, x, skip)) return;
-    const float sk = rgrad[t];
+    if (SKIP && in_deep(z, x, skip)) return;
     atomicAdd(lam + f, sk);
     if (seis::interior(z, x, g)) {
       const float Lu = lap5(um + b * g.plane, z, x, i, g, k.ih2);
@@ -1509,6 +1510,15 @@ __global__ __launch_bounds__(256) void k_habc_sum(const float* __restrict__ gpar
 }
 
 inline unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
+
+// The fused adjoint step with the rebuilt field over the old one, and the frame's
+// steps of the marching loops with either.
+template <int S, int VX>
+constexpr auto* k_habc_adj_in = &k_habc_adj_deep<S, VX, true>;
+template <int S>
+constexpr auto* k_frame_adj_in = &k_habc_adj_deep<S, 1, true>;
+template <int S>
+constexpr auto* k_frame_adj_out = &k_habc_adj_deep<S, 1, false>;
 
 #define SEIS_HABC_LAUNCH(K, S, grid, s, ...)                      \
   do {                                                            \
@@ -1608,6 +1618,20 @@ TileMap side_tiles(const Grid& g, const Deep& dp, int groups) {
   return m;
 }
 
+// Shot groups per frame thread: enough threads (about 400 thousand) come before
+// sharing the set-up per cell.  us per step, forward / adjoint, of the marching
+// loops' frame launches with groups of two shots: 300 x 500 x 8 1 group 10.7 / 38, 2
+// 11.6 / 41, 4 15.3 / 51; 900 x 2500 x 4 1 group 20.4 / 72, 2 20.0 / 68; x 16 1 group 75.6 /
+// 202, 2 70.1 / 179, 4 69.9 / 167, 8 72.5 / 177.  One step per launch, groups of four
+// shots, all in one thread and by this rule: 242 x 300 x 7 13.1 / 39.7 and 10.0 / 35.1,
+// 300 x 500 x 8 15.1 / 46.7 and 11.3 / 38.2, 313 x 344 x 13 20.1 / 60.8 and 12.3 / 42.6.
+// The adjoint's bands, whose set-up is longer, take twice as many: 451 x 877 x 4 37.2
+// for 39.1, 300 x 500 x 8 37.7 for 38.7.
+inline int frame_groups(int64_t nz, int64_t nx, int G, int most) {
+  const int64_t threads = 2 * (kW + 3) * (nz + nx) * G;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(most, (threads + 200000) / 400000));
+}
+
 // ---- four time steps per launch away from the boundary
 
 // Core: the cells at least kW + 3 + kMaxT from every edge.  Within kMaxT cells of
@@ -1632,16 +1656,6 @@ inline Deep shrunk(const Deep& c, int e) { return Deep{c.z0 + e, c.z1 - e, c.x0 
 // What a launch's adjoint sources reach of Core: a source in the frame kMaxT - 1
 // cells away is in Core's last level.
 inline Deep reach_of(const Deep& core) { return shrunk(core, 1 - kMaxT); }
-
-// Shot groups per thread of the frame's steps: a launch of its own needs enough
-// threads (about 400 thousand) before the set-up per cell is worth sharing.  us per
-// step, forward / adjoint, with groups of two shots: 300 x 500 x 8 1 group 10.7 / 38, 2
-// 11.6 / 41, 4 15.3 / 51; 900 x 2500 x 4 1 group 20.4 / 72, 2 20.0 / 68; x 16 1 group 75.6 /
-// 202, 2 70.1 / 179, 4 69.9 / 167, 8 72.5 / 177.
-inline int frame_groups(int64_t nz, int64_t nx, int G) {
-  const int64_t threads = 2 * kCoreMargin * (nz + nx) * G;
-  return (int)std::max<int64_t>(1, std::min<int64_t>(4, (threads + 200000) / 400000));
-}
 
 // row_slot[z] = 0 for every row that holds a receiver in `in` (-1 before).
 __global__ __launch_bounds__(256) void k_core_rows(const int64_t* __restrict__ rec, int64_t R,
@@ -1870,7 +1884,7 @@ int seis_habc_forward(const float* vp, const float* b, const float* wavelet, int
   const Grid gd{dp.z1 - dp.z0, dp.x1 - dp.x0, 0, (int64_t)(dp.z1 - dp.z0) * (dp.x1 - dp.x0)};
   const int G = (int)((B + S - 1) / S);
   const TileMap tmd = make_tiles(gd, VX, 1, G);
-  const int ngf = G < kFrameGroups ? G : kFrameGroups;  // groups per frame thread
+  const int ngf = std::min(G, frame_groups(nz, nx, G, kFrameGroups));
   const Frame fr = make_frame(g, dp, (G + ngf - 1) / ngf);
   const seis::TimeConsts k = seis::make_consts(dt, h);
   hipStream_t s = (hipStream_t)stream;
@@ -2126,9 +2140,9 @@ int seis_habc_backward(const float* vp, const float* b, const float* wavelet, in
   if (dp.x1 <= dp.x0 || dp.z1 <= dp.z0) dp = Deep{0, 0, 0, 0};  // no deep cells
   const Grid gd{dp.z1 - dp.z0, dp.x1 - dp.x0, 0, (int64_t)(dp.z1 - dp.z0) * (dp.x1 - dp.x0)};
   const TileMap tmd = make_tiles(gd, VX, kHabcRZ, G);
-  const int ngf = G < kFrameGroups ? G : kFrameGroups;  // groups per frame thread
+  const int ngf = std::min(G, frame_groups(nz, nx, G, kFrameGroups));
   const Frame fr = make_frame(g, dp, (G + ngf - 1) / ngf, true);
-  const int ngb = G < kBandGroups ? G : kBandGroups;  // groups per band thread
+  const int ngb = std::min(G, std::min(kBandGroups, 2 * ngf));
   const TileMap tmb = band_tiles(g, dp, kBandVX, (G + ngb - 1) / ngb);
   const TileMap tms = side_tiles(g, dp, (G + ngb - 1) / ngb);
   SEIS_CHECK_ARG(tms.per == 0 || (dp.x0 <= kLanes && (int)nx - dp.x1 <= kLanes),
@@ -2150,15 +2164,15 @@ int seis_habc_backward(const float* vp, const float* b, const float* wavelet, in
   for (int64_t kk = nt; kk >= 1; --kk) {
     const int recon = kk >= 3 ? 1 : (kk == 2 ? 2 : 0);
     SEIS_PROF(SEIS_KERNEL_HABC_BWD, s);
-    SEIS_HABC_LAUNCH_V(k_habc_adj_deep, S, VX,
+    SEIS_HABC_LAUNCH_V(k_habc_adj_in, S, VX,
                        dim3((tmd.per + fr.per + tmb.per + tms.per) * kXcds), s, vp, b, L1, L2,
-                       L0, X, Y, Y, grad_part, src_zx, wavelet + (kk - 1), recon, (int)B, hc, k,
+                       L0, X, Y, nullptr, grad_part, src_zx, wavelet + (kk - 1), recon, (int)B, hc, k,
                        dp, tmd, fr, ngf, G, tmb, ngb, tms);
     SEIS_PROF(SEIS_KERNEL_HABC_BWD, s);
     const int64_t work = R + (recon ? B * ring_len : 0);
     if (work > 0) {
       const float* slot = recon == 1 ? ring + (kk - 3) * B * ring_len : nullptr;
-      k_habc_post<<<nblk(work), 256, 0, s>>>(vp, X, Y, L0, grad_part, rec_flat,
+      k_habc_post<false><<<nblk(work), 256, 0, s>>>(vp, X, Y, L0, grad_part, rec_flat,
                                              R ? rec_grad + (kk - 1) * R : nullptr, R, slot,
                                              ring_len, recon, (int)B, S, g, k, Deep{0, 0, 0, 0});
       SEIS_CHECK_LAUNCH();
@@ -2224,7 +2238,7 @@ int seis_habc_march_forward(const float* vp, const float* b, const float* wavele
   const HabcCtx hc{seis::make_grid(nz, nx, npml, multiple != 0), multiple ? 1 : 0, dt, h};
   const Grid& g = hc.g;
   const int S = shots_per_group, G = (int)((B + S - 1) / S);
-  const int ngf = frame_groups(nz, nx, G);
+  const int ngf = frame_groups(nz, nx, G, 4);
   const Deep core = core_of(nz, nx);
   const Plan pl = make_plan(B * (core.z1 - core.z0) * (core.x1 - core.x0), widest(nx), 0, vec_x,
                             rows);
@@ -2347,7 +2361,7 @@ int seis_habc_march_backward(const float* vp, const float* b, const float* wavel
   const HabcCtx hc{seis::make_grid(nz, nx, npml, multiple != 0), multiple ? 1 : 0, dt, h};
   const Grid& g = hc.g;
   const int S = shots_per_group, G = (int)((B + S - 1) / S);
-  const int ngf = frame_groups(nz, nx, G), ngb = ngf;
+  const int ngf = frame_groups(nz, nx, G, 4), ngb = std::min(G, std::min(4, 2 * ngf));
   const Deep core = core_of(nz, nx);
   const Plan pl = make_plan(B * (core.z1 - core.z0) * (core.x1 - core.x0), widest(nx), 0, vec_x,
                             rows);
@@ -2439,13 +2453,19 @@ int seis_habc_march_backward(const float* vp, const float* b, const float* wavel
       const Frame fr = make_frame(g, dp, (G + ngf - 1) / ngf, true);
       const TileMap tmb = band_tiles(g, dp, kBandVX, (G + ngb - 1) / ngb);
       const TileMap tms = side_tiles(g, dp, (G + ngb - 1) / ngb);
-      SEIS_HABC_LAUNCH_V(k_habc_adj_deep, S, 1, dim3((fr.per + tmb.per + tms.per) * kXcds), s, vp,
-                         b, L[t], L[t - 1], L[t + 1], U[t], U[t - 1], U[t + 1], grad_part, src_zx,
-                         wavelet + (kt - 1), recon, (int)B, hc, k, dp, (TileMap{0, 0, 0, 0}), fr,
-                         ngf, G, tmb, ngb, tms);
+      const dim3 grid((fr.per + tmb.per + tms.per) * kXcds);
+      const TileMap none{0, 0, 0, 0};
+      if (U[t - 1] == U[t + 1])
+        SEIS_HABC_LAUNCH(k_frame_adj_in, S, grid, s, vp, b, L[t], L[t - 1], L[t + 1], U[t],
+                         U[t - 1], nullptr, grad_part, src_zx, wavelet + (kt - 1), recon, (int)B,
+                         hc, k, dp, none, fr, ngf, G, tmb, ngb, tms);
+      else
+        SEIS_HABC_LAUNCH(k_frame_adj_out, S, grid, s, vp, b, L[t], L[t - 1], L[t + 1], U[t],
+                         U[t - 1], U[t + 1], grad_part, src_zx, wavelet + (kt - 1), recon, (int)B,
+                         hc, k, dp, none, fr, ngf, G, tmb, ngb, tms);
       const int64_t items = R + B * ring_len;
       const float* slot = recon == 1 ? ring + (kt - 3) * B * ring_len : nullptr;
-      k_habc_post<<<nblk(items), 256, 0, s>>>(vp, U[t], U[t + 1], L[t + 1], grad_part, rec_flat,
+      k_habc_post<true><<<nblk(items), 256, 0, s>>>(vp, U[t], U[t + 1], L[t + 1], grad_part, rec_flat,
                                               R ? rec_grad + (kt - 1) * R : nullptr, R, slot,
                                               ring_len, recon, (int)B, S, g, k, dp);
       SEIS_CHECK_LAUNCH();

@@ -64,12 +64,13 @@ def _time_step_backward_multiple(*args, **kwargs):
 
 def _march_fits(B, nz, nx):
     """Whether the marching loops take the grid and pay for their launches of the
-    frame's steps.  us per step, forward / adjoint, one step per launch and
-    marching: 164 x 164 x 1 shot 6.4 / 24 and 6.5 / 26, 300 x 500 x 2 8.0 / 31 and
-    8.1 / 33, 900 x 2500 x 1 10.7 / 38 and 11.7 / 38, 300 x 500 x 8 15 / 50 and 10.7 /
-    38, 451 x 877 x 4 11.6 / 41 and 10.8 / 39, 900 x 2500 x 4 22 / 65 and 20 / 67, x
-    16 105 / 261 and 70 / 167."""
-    return B >= 4 and B * nz * nx >= 1000000 and bool(_lib.load().seis_habc_march_fits(nz, nx))
+    frame's steps: beyond what the last-level cache holds of five fields (about 12
+    10^6 cells).  us per step, forward / adjoint, one step per launch and marching:
+    164 x 164 x 1 shot 6.3 / 24 and 6.5 / 25, 900 x 2500 x 1 10.7 / 38 and 11.7 / 38, 313
+    x 344 x 13 12.3 / 43 and 11.6 / 45, 300 x 500 x 40 23 / 72 and 25 / 72, 900 x 2500 x 4
+    22 / 64 and 20 / 68, x 6 34 / 124 and 31 / 87, x 8 38 / 145 and 40 / 105, x 16 109 /
+    263 and 70 / 168."""
+    return B >= 4 and B * nz * nx >= 12000000 and bool(_lib.load().seis_habc_march_fits(nz, nx))
 
 
 def _march_rows(rec_flat, nz, nx):
@@ -151,6 +152,7 @@ class HabcLoop(torch.autograd.Function):
         bufs = _march_buffers(vp, rows, R, B, 5) if rows else None
         # the marching loops' frame steps in pairs of shots
         S = min(B, 2) if bufs else int(shots_per_group or default_shots_per_group(B))
+        u = None if bufs else [torch.empty((B, nz, nx), device=vp.device) for _ in range(3)]
         rec = torch.empty((nt, R), device=vp.device)
         ring = snaps = None
         K = 0
@@ -168,7 +170,6 @@ class HabcLoop(torch.autograd.Function):
                                B, dt, h, multiple, S)
             bufs = None
         else:
-            u = [torch.empty((B, nz, nx), device=vp.device) for _ in range(3)]
             _lib.call("seis_habc_forward", _lib.ptr(vp), _lib.ptr(b), _lib.ptr(wavelet), nt,
                       _lib.ptr(src_zx), _lib.ptr(rec_flat), R, _lib.ptr(rec), _lib.ptr(ring),
                       _lib.ptr(snaps), K, _lib.ptr(illum), _lib.ptr(u[0]), _lib.ptr(u[1]),
@@ -193,13 +194,14 @@ class HabcLoop(torch.autograd.Function):
         R = rec_flat.shape[0]
         G = (B + S - 1) // S
         grad_rec = grad_rec.contiguous().float()
-        gpart = torch.empty((G, nz, nx), device=vp.device)
         bufs = _march_buffers(vp, rows, R, B, 8) if rows else None
         if bufs is not None:
+            gpart = torch.empty((G, nz, nx), device=vp.device)
             grad = _march_backward(*bufs, vp, b, wavelet, src_zx, rec_flat, rows, grad_rec, ring,
                                    snaps, K, u_a, u_b, gpart, B, dt, h, multiple, S)
             return (grad,) + (None,) * 11
         lam = [torch.empty_like(u_a) for _ in range(3)]
+        gpart = torch.empty((G, nz, nx), device=vp.device)
         grad = torch.empty_like(vp)
         _lib.call("seis_habc_backward", _lib.ptr(vp), _lib.ptr(b), _lib.ptr(wavelet), nt,
                   _lib.ptr(src_zx), _lib.ptr(rec_flat), R,
