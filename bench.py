@@ -25,18 +25,19 @@ HELD_OUT_SEED = 20240611  # generator stream of the preconditioner's held-out pa
 HBM_PEAK = 8.0e12  # B/s, MI355X
 # algorithmic bytes per cell-update of each timed kernel (fields touched once
 # per step, damping/coefficients read once per cell)
-# (k_fwd2 advances two steps per launch, k_march_fwd and k_march_adj four:
-# their figures are per cell of a launch)
+# (k_fwd2 advances two steps per launch, k_march_fwd and k_march_adj four, the
+# HABC loops four with their frame's steps and k_el_fwd three: their figures are
+# per cell of a launch; the batched marching kernels' are per cell-update)
 BYTES_PER_CELL = {"k_fwd": 16.0, "k_bwd": 36.0, "k_fwd2": 32.0, "k_bwd2": 72.0,
                   "k_march_fwd": 16.0, "k_march_adj": 40.0,
-                  "k_habc_fwd": 16.0, "k_habc_adj": 36.0,
-                  "k_el_fwd": 52.0, "k_el_bwd": 116.0,
-                  "k_fwd_batch": 16.0, "k_fwd2_batch": 32.0, "k_bwd_batch": 36.0}
+                  "k_habc_fwd": 16.0, "k_habc_adj": 40.0,
+                  "k_el_fwd": 43.0, "k_el_bwd": 116.0,
+                  "k_march_fwd_batch": 4.0, "k_march_adj_batch": 10.0}
 KERNEL_IDS = {"acoustic": (("k_fwd", 0), ("k_bwd", 1), ("k_fwd2", 8), ("k_bwd2", 9),
                            ("k_march_fwd", 11), ("k_march_adj", 12)),
               "habc": (("k_habc_fwd", 4), ("k_habc_adj", 5)),
               "elastic": (("k_el_fwd", 2), ("k_el_bwd", 3)),
-              "generator": (("k_fwd2_batch", 6), ("k_bwd_batch", 7))}  # slot 6: the batched forward, two steps per launch
+              "generator": (("k_march_fwd_batch", 6), ("k_march_adj_batch", 7))}
 
 
 def parse():
@@ -304,7 +305,7 @@ def run_generator(args, dev):
     / its wall time, as for the single-model workloads."""
     import ctypes
     import torch
-    from seistorch_amd import _lib, autotune, generator
+    from seistorch_amd import _lib, generator
     t0 = time.perf_counter()
     spec = generator.GenSpec(n_models=args.models)
     host = generator.make_instances(spec=spec)
@@ -316,9 +317,7 @@ def run_generator(args, dev):
     cells = generator.cell_updates(host)
     print(f"[bench] generator: {len(host)} models, {cells:.3e} cell-updates per propagation, "
           f"built in {time.perf_counter() - t0:.1f} s", file=sys.stderr, flush=True)
-    shape, tune = autotune.tune_batch(generator.batch_instances(insts, "vp_start"))
-    launch = dict(shots_per_group=shape[0], rows_per_thread=shape[1], vec_x=shape[2])
-    print(f"[bench] autotuned batch launch shape {shape}", file=sys.stderr, flush=True)
+    launch = {}  # the marching loops choose their own launch shape
     use_graph = bool(args.graph)
     lib = _lib.load()
 
@@ -357,21 +356,21 @@ def run_generator(args, dev):
     if not use_graph:
         # per launch the batched kernels cover every running instance; the
         # algorithmic bytes of all timed launches over their summed duration
-        tot_ms, n_launch = kern["k_bwd_batch"]
-        achieved = BYTES_PER_CELL["k_bwd_batch"] * cells * args.steps / (tot_ms / 1e3)
+        tot_ms, n_launch = kern["k_march_adj_batch"]
+        achieved = BYTES_PER_CELL["k_march_adj_batch"] * cells * args.steps / (tot_ms / 1e3)
         # measured HBM bytes per cell-update (rocprof counters) x the average
         # cell-updates of one launch
         traffic = None
         tpath = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
                              "traffic.json")
-        per_cell = json.load(open(tpath)).get("k_bwd_batch_bytes_per_cell") \
+        per_cell = json.load(open(tpath)).get("k_march_adj_batch_bytes_per_cell") \
             if os.path.exists(tpath) else None
         if per_cell and n_launch:
             traffic = round(per_cell * cells * args.steps / n_launch)
-        roof = {"bound": "hbm", "kernel": "k_bwd_batch", "achieved": round(achieved / 1e9, 1),
+        roof = {"bound": "hbm", "kernel": "k_march_adj_batch", "achieved": round(achieved / 1e9, 1),
                 "peak": HBM_PEAK / 1e9, "unit": "GB/s", "frac": round(achieved / HBM_PEAK, 4),
                 "traffic": traffic, "avg_launch_us": round(tot_ms / max(n_launch, 1) * 1e3, 2),
-                "launches": n_launch, "bytes_per_cell_update": BYTES_PER_CELL["k_bwd_batch"]}
+                "launches": n_launch, "bytes_per_cell_update": BYTES_PER_CELL["k_march_adj_batch"]}
     out = {
         "metric": METRIC, "value": round(value, 3), "unit": "Gcell-updates/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup,
@@ -389,10 +388,7 @@ def run_generator(args, dev):
         "records_s_per_step": round(t_fwd / args.steps, 3),
         "roofline": roof,
         "kernels_ms_total": {k: round(v[0], 2) for k, v in kern.items()},
-        "launch_shape": {"shots_per_group": shape[0], "rows_per_thread": shape[1],
-                         "vec_x": shape[2],
-                         "autotune_ms": {f"S{a}_rz{b}_vx{c}": round(v, 2)
-                                         for (a, b, c), v in tune.items()}},
+        "launch_shape": None,
         "loss_sum": float(loss.sum()),
     }
     if args.copy_calibration:
@@ -788,9 +784,6 @@ def main():
         shape, tune = autotune.tune_elastic(P["vp_init"], P["vs_init"], P["rho_init"], P["d"],
                                             P["w"], P["src"], P["rec"], P["B"], P["dt"], P["h"],
                                             src_type=("txx", "tzz"), rec_type=("vx", "vz"))
-    elif args.workload == "habc":
-        shape, tune = autotune.tune_habc(P["vp_init"], P["b"], P["w"], P["src"], P["rec"], P["B"],
-                                         P["dt"], P["h"])
     if shape is not None:
         print(f"[bench] autotuned launch shape {shape}", file=sys.stderr, flush=True)
     for i in range(args.warmup):
