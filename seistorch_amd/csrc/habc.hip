@@ -147,11 +147,11 @@ __device__ __forceinline__ bool in_deep(int z, int x, const Deep& dp) {
   return z >= dp.z0 && z < dp.z1 && x >= dp.x0 && x < dp.x1;
 }
 
-// Shot groups per frame thread: the per-cell set-up of the strips runs once
-// per kFrameGroups groups of S shots.
+// Most shot groups per frame thread (see frame_groups): the per-cell set-up of the
+// strips runs once for them.
 constexpr int kFrameGroups = 8;
 
-// Shot groups per thread of the adjoint's top and bottom bands.
+// Most shot groups per thread of the adjoint's top and bottom bands.
 constexpr int kBandGroups = 8;
 
 // Cells per lane on the adjoint's bands: one, which divides every Deep lane

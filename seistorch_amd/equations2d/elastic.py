@@ -246,8 +246,9 @@ def propagate(vp, vs, rho, d, wavelet, src_zx, rec_flat, B, dt, h, src_type=("tx
     """Records (nt, R, nch) of B shots; differentiable w.r.t. vp, vs, rho.
     shots_per_group: shots per thread (1, 2, 4, 8), or a pair (forward,
     adjoint); None: the tuned value for this shape, else a default.
-    fused: each forward step and each reverse step of the adjoint in one pass
-    (five more field buffers).  illum: None, or an (nz, nx) float32 tensor
+    fused: up to three forward steps per launch (one with shots_per_group, the
+    illumination, or receivers on many grid rows) and each reverse step of the
+    adjoint in one pass (five more field buffers).  illum: None, or an (nz, nx) float32 tensor
     filled with the source illumination of the last source type's field
     (rnn.py:204-205).  multiple: free surface (d from
     ``pml.generate_pml_coefficients_2d(..., multiple=True)``); the gradients
