@@ -42,55 +42,16 @@ __device__ __forceinline__ bf16x8 load8(const uint16_t* p) {
 
 __device__ __forceinline__ bf16x8 zero8() { return __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0)); }
 
-// Phi(v) = (1 + erf(v / sqrt 2)) / 2.  Polynomials fitted here (least squares,
-// reweighted towards the smallest largest error): for |v| < 3, where nearly all
-// pre-activations lie, v times one in v^2; beyond, exp(-v^2 / 2) times one in
-// t = 1 / (1 + p |v|), which a wave skips when none of its lanes needs it.  For the
-// backward pass, where erff would cost two to three times as much.  Against 64
-// bits (rms): v Phi(v) 1.3e-8 for |v| < 1, 3.6e-8 to 2, 6.5e-8 to 9; with a
-// correctly rounded erf 1.4e-8, 3.6e-8, 7.2e-8.
-__device__ __forceinline__ float normal_cdf(float v, float v2) {
-  const float w = __fmaf_rn(v2, 2.222222239e-01f, -1.0f);
-  float q = 2.288580845e-06f;
-  q = __fmaf_rn(q, w, -1.250463993e-05f);
-  q = __fmaf_rn(q, w, 5.257648809e-05f);
-  q = __fmaf_rn(q, w, -2.172099921e-04f);
-  q = __fmaf_rn(q, w, 8.176510455e-04f);
-  q = __fmaf_rn(q, w, -2.729539294e-03f);
-  q = __fmaf_rn(q, w, 8.021571673e-03f);
-  q = __fmaf_rn(q, w, -2.057105117e-02f);
-  q = __fmaf_rn(q, w, 4.597223550e-02f);
-  q = __fmaf_rn(q, w, -9.283248335e-02f);
-  q = __fmaf_rn(q, w, 2.277131677e-01f);
-  float phi = __fmaf_rn(v, q, 0.5f);
-  if (!(fabsf(v) < 3.0f)) {
-    const float t = __builtin_amdgcn_rcpf(__fmaf_rn(fabsf(v), 2.262741625e-01f, 1.0f));
-    float p = -3.940436617e-02f;
-    p = __fmaf_rn(p, t, 1.016590074e-01f);
-    p = __fmaf_rn(p, t, -4.598595202e-02f);
-    p = __fmaf_rn(p, t, 8.938039094e-02f);
-    p = __fmaf_rn(p, t, 4.907613620e-02f);
-    p = __fmaf_rn(p, t, 7.944227010e-02f);
-    p = __fmaf_rn(p, t, 8.525198698e-02f);
-    p = __fmaf_rn(p, t, 9.029889852e-02f);
-    p = __fmaf_rn(p, t, 9.026946872e-02f);
-    const float h = t * p * __builtin_amdgcn_exp2f(-0.72134752044f * v2);
-    phi = v < 0.0f ? h : 1.0f - h;
-  }
-  return phi;
-}
-
 constexpr float kInvSqrt2 = 0.70710678118654752f;
+constexpr float kInvSqrt2Pi = 0.39894228040143268f;
 
-// The network's activation, erff's for the last place: see k_conv3x3_fwd.
-__device__ __forceinline__ float gelu_erf(float v) {
-  return 0.5f * v * (1.0f + erff(v * kInvSqrt2));
-}
+// The activation and its derivative by the library's functions, forward and
+// backward alike: both stand in front of a rounding to bf16 that every later layer
+// builds on, and another last place of either is another rounding here and there.
+__device__ __forceinline__ float gelu(float v) { return 0.5f * v * (1.0f + erff(v * kInvSqrt2)); }
 
 __device__ __forceinline__ float gelu_grad(float v) {
-  const float v2 = v * v;
-  return __fmaf_rn(v * 0.39894228040143268f, __builtin_amdgcn_exp2f(-0.72134752044f * v2),
-                   normal_cdf(v, v2));
+  return 0.5f * (1.0f + erff(v * kInvSqrt2)) + v * kInvSqrt2Pi * expf(-0.5f * v * v);
 }
 
 // Eight bf16 values as floats and back.
@@ -136,27 +97,16 @@ struct ConvInput {
 
 // ---------------------------------------------------------------- conv 3x3
 
-// Implicit GEMM on v_mfma_f32_16x16x32_bf16, weights as the first operand, so
-// that a lane ends with consecutive channels of one pixel.  A block of WAVES
-// waves computes (WAVES * RW) x 32 pixels x NT output channels, wave w the rows
-// w * RW on.  Per chunk of 32 input channels the (rows + 2) x 34 pixel window and
-// the 9 x NT x 32 weights go to LDS by asynchronous loads, into one buffer: what
-// hides their latency is the other blocks on the CU, three or more of them.  (Two
-// buffers, and persistent blocks that load the next tile meanwhile, leave room
-// for one block and were slower: 800 x 2400 pixels, 32 -> 32 channels 91 us, 100 x
-// 300, 256 -> 256 80 us.)  A wave reads each window row's fragment once per
-// horizontal tap and uses it for the output rows it reaches.
-//
-// LDS holds a pixel's (or weight row's) 32 channels as four 16-byte units, unit
-// u of window column c at slot u ^ ((c >> 2) & 3): 16 consecutive pixels then
-// read 16 distinct quarter-rows of banks, and the swizzle is the same in every
-// row, so that a lane needs one address per horizontal tap.  Weight rows are permuted, row j * 16 + m
-// holding channel (m / 4) * (NT / 4) + 4 * j + m % 4, so that a lane's NT / 4
-// results are consecutive channels and leave in 16-byte stores.
-//
-// MODE 1: y = acc (+ bias) in FP32; MODE 2: y = bf16(acc * gelu'(z)), the data
-// gradient taken through the activation before it.  (MODE 0, the forward pass, is
-// k_conv3x3_fwd.)
+// Every convolution, of the network or of its data gradient, sums an output's
+// products in the order k = tap * C + ci, 32 at a time, whatever the tile, so that
+// the bf16 activations and gradients depend on neither launch shape nor kernel.  (A
+// last-place difference before a rounding to bf16 is a different value for every
+// later layer: over the network's depth two orders drift apart by as much as either
+// is from the exact result, the training gradient by 1e-4 of its norm.)
+
+// kConvAct: z = acc + bias (bf16, optional) and y = act(z) (bf16).  kConvF32: yf = acc
+// (+ bias).  kConvGeluGrad: y = bf16(acc * gelu'(z)), the data gradient taken through
+// the activation before it.
 enum { kConvAct = 0, kConvF32 = 1, kConvGeluGrad = 2 };
 constexpr int kTileW = 32;
 constexpr int kWinW = kTileW + 2;
@@ -167,24 +117,80 @@ struct ConvArgs {
   int N, H, W;
   const uint16_t* w;
   const float* bias;
-  int Cout, vec;  // vec: Cout % 8 == 0 and 16-byte aligned outputs
-  uint16_t* z;  // MODE 2: the activation's input (read)
-  uint16_t* y;
+  int Cout, act;
+  uint16_t *z, *y;  // kConvGeluGrad reads z
   float* yf;
-  int tx, ty, ntile, per;  // tiles in x and y, output-channel tiles, tiles per XCD
+  int vec;  // Cout % 8 == 0 and 16-byte aligned outputs
+  int tx, ty, ntile, per, lg;  // tiles in x and y, output-channel tiles, tiles per XCD
 };
 
-template <int WAVES, int RW, int NT, int MODE>
-__global__ __launch_bounds__(WAVES * 64) void k_conv3x3(ConvArgs a) {
+// A pixel's M sums, of the channels from cb on: bias, activation, stores at o.
+template <int MODE, int M>
+__device__ __forceinline__ void conv_out(const ConvArgs& a, int64_t o, int cb,
+                                         const float (&v)[M]) {
+#pragma unroll
+  for (int h = 0; h < M; h += 8) {
+    if (cb + h + 8 <= a.Cout && a.vec) {
+      float y[8], t[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = v[h + e];
+      if constexpr (MODE == kConvF32) {
+        *reinterpret_cast<float4*>(a.yf + o + h) = make_float4(y[0], y[1], y[2], y[3]);
+        *reinterpret_cast<float4*>(a.yf + o + h + 4) = make_float4(y[4], y[5], y[6], y[7]);
+      } else if constexpr (MODE == kConvGeluGrad) {
+        unpack8(a.z + o + h, t);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] *= gelu_grad(t[e]);
+        pack8(a.y + o + h, y);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t[e] = a.act ? gelu(y[e]) : y[e];
+        if (a.z) pack8(a.z + o + h, y);
+        pack8(a.y + o + h, t);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (cb + h + e >= a.Cout) continue;
+        const float y = v[h + e];
+        const int64_t q = o + h + e;
+        if constexpr (MODE == kConvF32) {
+          a.yf[q] = y;
+        } else if constexpr (MODE == kConvGeluGrad) {
+          a.y[q] = f2bf(y * gelu_grad(bf2f(a.z[q])));
+        } else {
+          if (a.z) a.z[q] = f2bf(y);
+          a.y[q] = f2bf(a.act ? gelu(y) : y);
+        }
+      }
+    }
+  }
+}
+
+// The data gradient of a layer with 32 output channels: implicit GEMM on
+// v_mfma_f32_16x16x32_bf16, weights as the first operand, so that a lane ends with
+// consecutive channels of one pixel.  A block of WAVES waves computes (WAVES * RW) x
+// 32 pixels x 32 channels, wave w the rows w * RW on.  The (rows + 2) x 34 pixel
+// window and the 9 x 32 x 32 weights go to LDS by asynchronous loads; what hides
+// their latency is the other blocks on the CU.  A wave holds the nine taps' weights
+// in registers and reads each fragment of a window row once for the output rows that
+// it reaches: the rows from above, so that each of them meets its taps in order.
+//
+// LDS holds a pixel's (or weight row's) 32 channels as four 16-byte units, unit
+// u of window column c at slot u ^ ((c >> 2) & 3): 16 consecutive pixels then
+// read 16 distinct quarter-rows of banks, and the swizzle is the same in every
+// row, so that a lane needs one address per horizontal tap.  Weight rows are permuted,
+// row j * 16 + m holding channel (m / 4) * 8 + 4 * j + m % 4, so that a lane's 8
+// results are consecutive channels and leave in 16-byte stores.
+template <int WAVES, int RW, int MODE>
+__global__ __launch_bounds__(WAVES * 64) void k_conv3x3_grad32(ConvArgs a) {
   constexpr int kThr = WAVES * 64, kRows = WAVES * RW, kPx = (kRows + 2) * kWinW;
-  constexpr int kAU = kPx * 4, kBU = 9 * NT * 4;  // 16-byte units of one buffer
+  constexpr int NT = 32, NF = 2, C = 32, K = 9 * C;
+  constexpr int kAU = kPx * 4, kBU = 9 * NT * 4;  // 16-byte units
   constexpr int kAP = (kAU + kThr - 1) / kThr, kBP = (kBU + kThr - 1) / kThr;
-  constexpr int kAS = kAP * kThr * kUnit, kBS = kBP * kThr * kUnit;
-  constexpr int NF = NT / 16;
-  __shared__ __align__(16) uint16_t sA[kAS];
-  __shared__ __align__(16) uint16_t sB[kBS];
+  __shared__ __align__(16) uint16_t sA[kAP * kThr * kUnit];
+  __shared__ __align__(16) uint16_t sB[kBP * kThr * kUnit];
   const int t = threadIdx.x, wave = t / 64, l = t % 64, m = l % 16, kq = l / 16;
-  const int C = a.in.C, K = 9 * C, nk = (C + 31) / 32;
   // XCD-aware order: the output-channel tiles of one pixel tile, then the next
   // pixel tile, on the same XCD
   const int unit = (int)(blockIdx.x % 8) * a.per + (int)(blockIdx.x / 8);
@@ -193,64 +199,31 @@ __global__ __launch_bounds__(WAVES * 64) void k_conv3x3(ConvArgs a) {
   const int px0 = (tile % a.tx) * kTileW, py0 = ((tile / a.tx) % a.ty) * kRows;
   const int n = tile / (a.tx * a.ty);
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-  // this thread's units of a window: pixel offset from the tile's first pixel in
-  // the image and in the half-size one, channel offset
-  int rx[kAP], rl[kAP], cu[kAP];
+  const uint16_t* x0 = a.in.x + (((int64_t)n * a.H + py0) * a.W + px0) * C;
+  // uniform: no unit lies outside the image or the channels
+  const bool inside = px0 > 0 && px0 + kTileW < a.W && py0 > 0 && py0 + kRows < a.H;
+  const bool whole = co0 + NT <= a.Cout;
 #pragma unroll
   for (int i = 0; i < kAP; ++i) {
     const int p = (i * kThr + t) / 4, r = p / kWinW - 1, c = p % kWinW - 1;
-    rx[i] = r * a.W + c;
-    rl[i] = (r >> 1) * (a.W / 2) + (c >> 1);
-    cu[i] = ((t & 3) ^ (((p % kWinW) >> 2) & 3)) * kUnit;
+    bool ok = true;
+    if (!inside) ok = py0 + r >= 0 && py0 + r < a.H && px0 + c >= 0 && px0 + c < a.W;
+    if (kAU % kThr != 0 && i == kAP - 1) ok = ok && p < kPx;
+    const int cu = ((t & 3) ^ (((c + 1) >> 2) & 3)) * kUnit;
+    if (ok) async16(x0 + ((int64_t)(r * a.W + c) * C + cu), &sA[(i * kThr + wave * 64) * kUnit]);
+    else *reinterpret_cast<uint4*>(&sA[(i * kThr + t) * kUnit]) = zero;
   }
-  auto fetch_x = [&](int kc) {
-    const int c0 = kc * 32;
-    const bool lo = c0 < a.in.C1;  // uniform: C1 is a multiple of 32
-    const int cs = lo ? a.in.C1 : C - a.in.C1, left = C - c0;
-    const uint16_t* src =
-        lo ? a.in.low + c0 + (((int64_t)n * (a.H / 2) + py0 / 2) * (a.W / 2) + px0 / 2) * cs
-           : a.in.x + (c0 - a.in.C1) + (((int64_t)n * a.H + py0) * a.W + px0) * cs;
-    const bool inside = px0 > 0 && px0 + kTileW < a.W && py0 > 0 && py0 + kRows < a.H &&
-                        left >= 32;  // uniform: nothing to zero
-#pragma unroll
-    for (int i = 0; i < kAP; ++i) {
-      const int p = (i * kThr + t) / 4;
-      bool ok = true;
-      if (!inside) {
-        const int yy = py0 + p / kWinW - 1, xx = px0 + p % kWinW - 1;
-        ok = yy >= 0 && yy < a.H && xx >= 0 && xx < a.W && cu[i] < left;
-      }
-      if (kAU % kThr != 0 && i == kAP - 1) ok = ok && p < kPx;
-      if (ok)
-        async16(src + ((int64_t)(lo ? rl[i] : rx[i]) * cs + cu[i]), &sA[(i * kThr + wave * 64) * kUnit]);
-      else *reinterpret_cast<uint4*>(&sA[(i * kThr + t) * kUnit]) = zero;
-    }
-  };
-  int wo[kBP];  // weight offset of this thread's units in the first output-channel tile
 #pragma unroll
   for (int i = 0; i < kBP; ++i) {
     const int u = i * kThr + t, row = (u / 4) % NT, tap = u / (4 * NT);
     const int cq = (t & 3) ^ ((row >> 2) & 3), j = row / 16, mm = row % 16;
-    wo[i] = ((mm / 4) * (NT / 4) + 4 * j + mm % 4) * K + tap * C + cq * kUnit;
+    const int co = co0 + (mm / 4) * 8 + 4 * j + mm % 4;
+    bool ok = whole || co < a.Cout;
+    if (kBU % kThr != 0 && i == kBP - 1) ok = ok && u < kBU;
+    uint16_t* to = &sB[(i * kThr + wave * 64) * kUnit];
+    if (ok) async16(a.w + (int64_t)co * K + tap * C + cq * kUnit, to);
+    else *reinterpret_cast<uint4*>(&sB[u * kUnit]) = zero;
   }
-  auto fetch_w = [&](int kc) {
-    const int c0 = kc * 32, left = C - c0;
-    const uint16_t* src = a.w + (int64_t)co0 * K + c0;
-    const bool whole = co0 + NT <= a.Cout && left >= 32;  // uniform
-#pragma unroll
-    for (int i = 0; i < kBP; ++i) {
-      const int u = i * kThr + t;
-      bool ok = true;
-      if (!whole) {
-        const int row = (u / 4) % NT, j = row / 16, mm = row % 16;
-        ok = co0 + (mm / 4) * (NT / 4) + 4 * j + mm % 4 < a.Cout &&
-             ((t & 3) ^ ((row >> 2) & 3)) * kUnit < left;
-      }
-      if (kBU % kThr != 0 && i == kBP - 1) ok = ok && u < kBU;
-      if (ok) async16(src + wo[i], &sB[(i * kThr + wave * 64) * kUnit]);
-      else *reinterpret_cast<uint4*>(&sB[u * kUnit]) = zero;
-    }
-  };
   floatx4 acc[RW][2][NF];
 #pragma unroll
   for (int r = 0; r < RW; ++r)
@@ -265,43 +238,36 @@ __global__ __launch_bounds__(WAVES * 64) void k_conv3x3(ConvArgs a) {
   for (int dx = 0; dx < 3; ++dx)
     xa[dx] = ((wave * RW * kWinW + m + dx) * 4 + (kq ^ (((m + dx) >> 2) & 3))) * kUnit;
   const int wa = (m * 4 + (kq ^ ((m >> 2) & 3))) * kUnit;
-  for (int kc = 0; kc < nk; ++kc) {
-    if (kc > 0) __syncthreads();  // the previous chunk has been read
-    fetch_x(kc);
-    fetch_w(kc);
-    lds_arrived();
-    __syncthreads();
+  lds_arrived();
+  __syncthreads();
+  bf16x8 wf[9][NF];
+#pragma unroll
+  for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+    for (int j = 0; j < NF; ++j) wf[tap][j] = load8(&sB[wa + (tap * NT + j * 16) * 4 * kUnit]);
+#pragma unroll
+  for (int ir = 0; ir < RW + 2; ++ir) {
 #pragma unroll
     for (int dx = 0; dx < 3; ++dx) {
-      bf16x8 wf[3][NF];
 #pragma unroll
-      for (int dy = 0; dy < 3; ++dy)
+      for (int f = 0; f < 2; ++f) {
+        const bf16x8 xf = load8(&sA[xa[dx] + (ir * kWinW + f * 16) * 4 * kUnit]);
 #pragma unroll
-        for (int j = 0; j < NF; ++j) {
-          wf[dy][j] = load8(&sB[wa + ((dy * 3 + dx) * NT + j * 16) * 4 * kUnit]);
-        }
+        for (int dy = 0; dy < 3; ++dy) {
+          const int r = ir - dy;
+          if (r < 0 || r >= RW) continue;
 #pragma unroll
-      for (int ir = 0; ir < RW + 2; ++ir) {
-#pragma unroll
-        for (int f = 0; f < 2; ++f) {
-          const bf16x8 xf = load8(&sA[xa[dx] + (ir * kWinW + f * 16) * 4 * kUnit]);
-#pragma unroll
-          for (int dy = 0; dy < 3; ++dy) {
-            const int r = ir - dy;
-            if (r < 0 || r >= RW) continue;
-#pragma unroll
-            for (int j = 0; j < NF; ++j)
-              acc[r][f][j] =
-                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[dy][j], xf, acc[r][f][j], 0, 0, 0);
-          }
+          for (int j = 0; j < NF; ++j)
+            acc[r][f][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[dy * 3 + dx][j], xf,
+                                                                   acc[r][f][j], 0, 0, 0);
         }
       }
     }
   }
-  const int cb = co0 + kq * (NT / 4);  // this lane's NT / 4 consecutive channels
-  float bv[NT / 4];
+  const int cb = co0 + kq * 8;  // this lane's 8 consecutive channels
+  float bv[8];
 #pragma unroll
-  for (int e = 0; e < NT / 4; ++e) bv[e] = a.bias && cb + e < a.Cout ? a.bias[cb + e] : 0.0f;
+  for (int e = 0; e < 8; ++e) bv[e] = a.bias && cb + e < a.Cout ? a.bias[cb + e] : 0.0f;
 #pragma unroll
   for (int r = 0; r < RW; ++r) {
     const int yy = py0 + wave * RW + r;
@@ -310,77 +276,31 @@ __global__ __launch_bounds__(WAVES * 64) void k_conv3x3(ConvArgs a) {
     for (int f = 0; f < 2; ++f) {
       const int xx = px0 + f * 16 + m;
       if (xx >= a.W) continue;
-      const int64_t o = (((int64_t)n * a.H + yy) * a.W + xx) * a.Cout + cb;
-      float v[NT / 4];
+      float v[8];
 #pragma unroll
-      for (int e = 0; e < NT / 4; ++e) v[e] = acc[r][f][e / 4][e % 4] + bv[e];
-      if (a.vec) {
-#pragma unroll
-        for (int h = 0; h < NT / 4; h += 8) {
-          if (cb + h >= a.Cout) continue;
-          if constexpr (MODE == kConvF32) {
-            *reinterpret_cast<float4*>(a.yf + o + h) =
-                make_float4(v[h], v[h + 1], v[h + 2], v[h + 3]);
-            *reinterpret_cast<float4*>(a.yf + o + h + 4) =
-                make_float4(v[h + 4], v[h + 5], v[h + 6], v[h + 7]);
-          } else {
-            float e8[8], z8[8];
-            unpack8(a.z + o + h, z8);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) e8[e] = v[h + e] * gelu_grad(z8[e]);
-            pack8(a.y + o + h, e8);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < NT / 4; ++e) {
-          if (cb + e >= a.Cout) continue;
-          if constexpr (MODE == kConvF32) {
-            a.yf[o + e] = v[e];
-          } else {
-            a.y[o + e] = f2bf(v[e] * gelu_grad(bf2f(a.z[o + e])));
-          }
-        }
-      }
+      for (int e = 0; e < 8; ++e) v[e] = acc[r][f][e / 4][e % 4] + bv[e];
+      conv_out<MODE, 8>(a, (((int64_t)n * a.H + yy) * a.W + xx) * a.Cout + cb, cb, v);
     }
   }
 }
 
-// ------------------------------------------------- conv 3x3 of the network
-
-// The network's own convolutions, z = conv + bias, y = act(z): every output sums
-// its products in the order k = tap * C + ci, 32 at a time, whatever the tile, so
-// the bf16 activations do not depend on the launch shape.  (k_conv3x3 takes the
-// channels 32 at a time and the taps inside: a last-place difference before a
-// rounding to bf16 is a different activation, and over the network's depth the
-// outputs of the two orders drift apart by as much as either is from the exact
-// result.)  With the taps outside, all C channels of the window have to be at
-// hand: a block of TH x TW pixels loads them once into LDS (asynchronously, C up
-// to 512) and its waves then run through all of K without a barrier.  What bounds
-// it is the latency of the weights' 64-byte rows from L2: 25 to 40 % of the matrix
-// rate at 96 channels and more, 15 % at 32.  Wave (wm,
-// wn) owns MR fragments of 16 pixels and 16 * NF output channels; the weights come
-// straight from L2, two steps ahead, into registers.
+// The network's own convolutions and the data gradient of wider layers.  With the
+// taps outside, all C channels of the window have to be at hand: a block of TH x TW
+// pixels loads them once into LDS (asynchronously, C up to 512) and its waves then run
+// through all of K without a barrier.  What bounds it is the latency of the weights'
+// 64-byte rows from L2: 25 to 40 % of the matrix rate at 96 channels and more, 15 % at
+// 32.  Wave (wm, wn) owns MR fragments of 16 pixels and 16 * NF output channels; the
+// weights come straight from L2, two steps ahead, into registers.
 //
 // Pixels lie C * 2 bytes apart; the 16-byte unit u of window column c is at u ^
 // ((c >> (4 - lg)) & (2^lg - 1)), 2^lg being the largest power of two in C / 8 (at
 // most 16): 16 neighbouring pixels then read from all banks.
-struct FwdConvArgs {
-  ConvInput in;
-  int N, H, W;
-  const uint16_t* w;
-  const float* bias;
-  int Cout, act;
-  uint16_t *z, *y;
-  int vec;  // Cout % 8 == 0 and 16-byte aligned outputs
-  int tx, ty, ntile, per, lg;
-};
 
 // kOne: C is 32, so that a step's 32 products are one tap.  kFar: C is beyond the
 // LDS; the fragments come straight from memory (no layer of the default network).
 enum { kAny = 0, kOne = 1, kFar = 2 };
-template <int TH, int TW, int MR, int NF, int WM, int WN, int KIND>
-__global__ __launch_bounds__(64 * WM * WN) void k_conv3x3_fwd(FwdConvArgs a) {
+template <int TH, int TW, int MR, int NF, int WM, int WN, int KIND, int MODE>
+__global__ __launch_bounds__(64 * WM * WN) void k_conv3x3(ConvArgs a) {
   static_assert(TH * TW == 16 * MR * WM, "the waves cover the tile");
   constexpr int kThr = 64 * WM * WN, kWin = TW + 2, kPx = (TH + 2) * kWin, kFx = TW / 16;
   constexpr int NT = 16 * NF;  // a wave's output channels
@@ -511,27 +431,10 @@ __global__ __launch_bounds__(64 * WM * WN) void k_conv3x3_fwd(FwdConvArgs a) {
   for (int r = 0; r < MR; ++r) {
     const int f = wm * MR + r, yy = py0 + f / kFx, xx = px0 + (f % kFx) * 16 + m;
     if (yy >= a.H || xx >= a.W) continue;
-    const int64_t o = (((int64_t)n * a.H + yy) * a.W + xx) * a.Cout + cb;
+    float v[NT / 4];
 #pragma unroll
-    for (int h = 0; h < NT / 4; h += 8) {
-      float zv[8], yv[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        zv[e] = acc[r][(h + e) / 4][e % 4] + bv[h + e];
-        yv[e] = a.act ? gelu_erf(zv[e]) : zv[e];
-      }
-      if (cb + h + 8 <= a.Cout && a.vec) {
-        if (a.z) pack8(a.z + o + h, zv);
-        pack8(a.y + o + h, yv);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          if (cb + h + e >= a.Cout) continue;
-          if (a.z) a.z[o + h + e] = f2bf(zv[e]);
-          a.y[o + h + e] = f2bf(yv[e]);
-        }
-      }
-    }
+    for (int e = 0; e < NT / 4; ++e) v[e] = acc[r][e / 4][e % 4] + bv[e];
+    conv_out<MODE, NT / 4>(a, (((int64_t)n * a.H + yy) * a.W + xx) * a.Cout + cb, cb, v);
   }
 }
 
@@ -1033,26 +936,24 @@ __global__ __launch_bounds__(256) void k_head_fwd(const uint16_t* __restrict__ x
   out[t] = s + b[0];
 }
 
-// k_head_fwd with G lanes of 8 channels per pixel (C = 8 * G), whose sums are
-// added across the lanes.
+// k_head_fwd with 16-byte loads (C = 8 * G); the channels in the same order, since the
+// training gradient's roundings follow from the output.
 template <int G>
 __global__ __launch_bounds__(256) void k_head_fwd_v(const uint16_t* __restrict__ x, int64_t P,
                                                     const float* __restrict__ w,
                                                     const float* __restrict__ b,
                                                     float* __restrict__ out) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t p = t / G;
-  const int c = (int)(t % G) * 8;
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= P) return;
+  float xv[G][8];
+#pragma unroll
+  for (int q = 0; q < G; ++q) unpack8(x + (p * G + q) * 8, xv[q]);
   float s = 0.0f;
-  if (p < P) {
-    float xv[8];
-    unpack8(x + p * 8 * G + c, xv);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) s += xv[e] * w[c + e];
-  }
+  for (int q = 0; q < G; ++q)
 #pragma unroll
-  for (int o = 1; o < G; o *= 2) s += __shfl_xor(s, o);
-  if (p < P && c == 0) out[p] = s + b[0];
+    for (int e = 0; e < 8; ++e) s += xv[q][e] * w[q * 8 + e];
+  out[p] = s + b[0];
 }
 
 // Head gradient taken through the last activation, 8 channels per thread and
@@ -1176,45 +1077,21 @@ inline unsigned blocks_for(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-template <int WAVES, int RW, int NT, int MODE>
-int launch_conv(ConvArgs a, hipStream_t s) {
-  a.tx = (a.W + kTileW - 1) / kTileW;
-  a.ty = (a.H + WAVES * RW - 1) / (WAVES * RW);
-  a.ntile = (a.Cout + NT - 1) / NT;
+int conv_grid(ConvArgs& a, int rows, int cols, int channels) {
+  a.tx = (a.W + cols - 1) / cols;
+  a.ty = (a.H + rows - 1) / rows;
+  a.ntile = (a.Cout + channels - 1) / channels;
   const int64_t units = (int64_t)a.N * a.ty * a.tx * a.ntile;
   SEIS_CHECK_ARG(units < ((int64_t)1 << 31) - 8, "too many tiles");
   a.per = (int)((units + 7) / 8);
-  k_conv3x3<WAVES, RW, NT, MODE><<<(unsigned)(a.per * 8), WAVES * 64, 0, s>>>(a);
-  SEIS_CHECK_LAUNCH();
   return 0;
 }
 
-// 8 or 4 rows of 32 pixels per block, 4 where the deep levels of the network
-// would leave CUs without two blocks; 16 rows where one chunk is the whole
-// reduction (the load is exposed once per block, so larger blocks win).  us for
-// the 800 x 2400 network's layers with 16 / 8 / 4 rows: 32 -> 32 channels 82 / 93 /
-// 95, 64 -> 64 62 / 61 / 66, 96 -> 32 175 / 171 / 195, 512 -> 256 101 / 87 / 97, 50 x
-// 150 pixels 256 -> 256 24 / 23 / 23, 16 x 24 x 8 images 24 / 19 / 15; 64 output
-// channels per block were slower at every layer but 384 -> 128 (106 for 111).
-template <int MODE>
-int pick_conv(const ConvArgs& a, hipStream_t s) {
-  const int64_t b8 = (int64_t)a.N * ((a.H + 7) / 8) * ((a.W + kTileW - 1) / kTileW) *
-                     ((a.Cout + 31) / 32);
-  if (b8 < 512) return launch_conv<4, 1, 32, MODE>(a, s);
-  if (a.in.C <= 32) return launch_conv<8, 2, 32, MODE>(a, s);
-  return launch_conv<4, 2, 32, MODE>(a, s);
-}
-
-template <int TH, int TW, int MR, int NF, int WM, int WN, int KIND = kAny>
-int launch_conv_fwd(FwdConvArgs a, hipStream_t s) {
-  a.tx = (a.W + TW - 1) / TW;
-  a.ty = (a.H + TH - 1) / TH;
-  a.ntile = (a.Cout + 16 * NF * WN - 1) / (16 * NF * WN);
-  const int64_t units = (int64_t)a.N * a.ty * a.tx * a.ntile;
-  SEIS_CHECK_ARG(units < ((int64_t)1 << 31) - 8, "too many tiles");
-  a.per = (int)((units + 7) / 8);
+template <int TH, int TW, int MR, int NF, int WM, int WN, int KIND, int MODE>
+int launch_conv(ConvArgs a, hipStream_t s) {
+  if (int e = conv_grid(a, TH, TW, 16 * NF * WN)) return e;
   const int lds = KIND == kFar ? 0 : (TH + 2) * (TW + 2) * a.in.C * 2;
-  auto* k = k_conv3x3_fwd<TH, TW, MR, NF, WM, WN, KIND>;
+  auto* k = k_conv3x3<TH, TW, MR, NF, WM, WN, KIND, MODE>;
   SEIS_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds));
   k<<<(unsigned)(a.per * 8), 64 * WM * WN, lds, s>>>(a);
@@ -1222,9 +1099,27 @@ int launch_conv_fwd(FwdConvArgs a, hipStream_t s) {
   return 0;
 }
 
-int pick_conv_fwd(FwdConvArgs a, hipStream_t s) {
+template <int WAVES, int RW, int MODE>
+int launch_grad32(ConvArgs a, hipStream_t s) {
+  if (int e = conv_grid(a, WAVES * RW, kTileW, 32)) return e;
+  k_conv3x3_grad32<WAVES, RW, MODE><<<(unsigned)(a.per * 8), WAVES * 64, 0, s>>>(a);
+  SEIS_CHECK_LAUNCH();
+  return 0;
+}
+
+template <int MODE>
+int pick_conv(ConvArgs a, hipStream_t s) {
   while (a.lg < 4 && (a.in.C / 8) % (2 << a.lg) == 0) ++a.lg;
   const int C = a.in.C;
+  if constexpr (MODE != kConvAct) {
+    // 16 rows of 32 pixels per block, 4 where small images would leave CUs without
+    // two blocks
+    if (C == 32) {
+      const int64_t b8 = (int64_t)a.N * ((a.H + 7) / 8) * ((a.W + kTileW - 1) / kTileW) *
+                         ((a.Cout + 31) / 32);
+      return b8 < 512 ? launch_grad32<4, 1, MODE>(a, s) : launch_grad32<8, 2, MODE>(a, s);
+    }
+  }
   // Tile and waves by what the window leaves of the LDS, the best of 14 shapes at
   // the layers of an 800 x 2400 image.  us, now and with blocks of one row of 64
   // pixels that reload their window per 32 channels: 32 -> 32 channels 159 and 200,
@@ -1232,15 +1127,17 @@ int pick_conv_fwd(FwdConvArgs a, hipStream_t s) {
   // 256 at an eighth 83 and 103, and with the concatenation's pass (676 MB written over
   // the four levels) before it 96 -> 32 301 and 480, 192 -> 64 264 and 295, 384 -> 128 285
   // and 314, 512 -> 256 164 and 209.
-  if (a.Cout <= 32 && C == 32) return launch_conv_fwd<8, 32, 4, 2, 4, 1, kOne>(a, s);
-  if (a.Cout <= 32 && C <= 128) return launch_conv_fwd<8, 32, 4, 2, 4, 1>(a, s);
-  if (C == 32) return launch_conv_fwd<4, 16, 4, 2, 1, 2, kOne>(a, s);
-  if (C <= 64) return launch_conv_fwd<4, 16, 4, 2, 1, 2>(a, s);
-  if (C <= 128 || (C > 192 && C <= 256)) return launch_conv_fwd<4, 16, 4, 2, 1, 4>(a, s);
-  if (C <= 192) return launch_conv_fwd<4, 32, 4, 2, 2, 2>(a, s);
-  if (C <= 384) return launch_conv_fwd<4, 32, 4, 4, 2, 2>(a, s);
-  if (C <= 512) return launch_conv_fwd<4, 16, 4, 4, 1, 4>(a, s);
-  return launch_conv_fwd<4, 16, 4, 4, 1, 4, kFar>(a, s);
+  if constexpr (MODE == kConvAct) {
+    if (a.Cout <= 32 && C == 32) return launch_conv<8, 32, 4, 2, 4, 1, kOne, MODE>(a, s);
+    if (C == 32) return launch_conv<4, 16, 4, 2, 1, 2, kOne, MODE>(a, s);
+  }
+  if (a.Cout <= 32 && C <= 128) return launch_conv<8, 32, 4, 2, 4, 1, kAny, MODE>(a, s);
+  if (C <= 64) return launch_conv<4, 16, 4, 2, 1, 2, kAny, MODE>(a, s);
+  if (C <= 128 || (C > 192 && C <= 256)) return launch_conv<4, 16, 4, 2, 1, 4, kAny, MODE>(a, s);
+  if (C <= 192) return launch_conv<4, 32, 4, 2, 2, 2, kAny, MODE>(a, s);
+  if (C <= 384) return launch_conv<4, 32, 4, 4, 2, 2, kAny, MODE>(a, s);
+  if (C <= 512) return launch_conv<4, 16, 4, 4, 1, 4, kAny, MODE>(a, s);
+  return launch_conv<4, 16, 4, 4, 1, 4, kFar, MODE>(a, s);
 }
 
 int conv(int mode, const ConvInput& in, int32_t N, int32_t H, int32_t W, const uint16_t* w,
@@ -1255,9 +1152,8 @@ int conv(int mode, const ConvInput& in, int32_t N, int32_t H, int32_t W, const u
   SEIS_CHECK_ARG(y || (!z && !act), "z and act apply to the bf16 output only");
   SEIS_CHECK_ARG((int64_t)N * H <= (int64_t)1 << 24, "too many image rows");
   const int vec = Cout % 8 == 0 && aligned16(z) && aligned16(y) && aligned16(yf);
-  if (mode == kConvAct)
-    return pick_conv_fwd({in, N, H, W, w, bias, Cout, act, z, y, vec, 0, 0, 0, 0, 0}, s);
-  const ConvArgs a{in, N, H, W, w, bias, Cout, vec, z, y, yf, 0, 0, 0, 0};
+  const ConvArgs a{in, N, H, W, w, bias, Cout, act, z, y, yf, vec, 0, 0, 0, 0, 0};
+  if (mode == kConvAct) return pick_conv<kConvAct>(a, s);
   if (mode == kConvF32) return pick_conv<kConvF32>(a, s);
   return pick_conv<kConvGeluGrad>(a, s);
 }
@@ -1527,7 +1423,7 @@ int seis_unet_head(const uint16_t* x, int64_t P, int32_t C, const float* w, cons
                    float* out, void* stream) {
   SEIS_CHECK_ARG(x && w && b && out && C >= 1, "bad arguments");
   if (C == 32 && aligned16(x))
-    k_head_fwd_v<4><<<blocks_for(4 * P), 256, 0, (hipStream_t)stream>>>(x, P, w, b, out);
+    k_head_fwd_v<4><<<blocks_for(P), 256, 0, (hipStream_t)stream>>>(x, P, w, b, out);
   else
     k_head_fwd<<<blocks_for(P), 256, 0, (hipStream_t)stream>>>(x, P, C, w, b, out);
   SEIS_CHECK_LAUNCH();
