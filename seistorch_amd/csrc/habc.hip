@@ -832,7 +832,7 @@ int seis_habc_forward(const float* vp, const float* b, const float* wavelet, int
   const Grid gd{dp.z1 - dp.z0, dp.x1 - dp.x0, 0, (int64_t)(dp.z1 - dp.z0) * (dp.x1 - dp.x0)};
   const int G = (int)((B + S - 1) / S);
   const TileMap tmd = make_tiles(gd, VX, 1, G);
-  const int ngf = std::min(G, frame_groups(nz, nx, G, kFrameGroups));
+  const int ngf = frame_groups(nz, nx, G, S);
   const Frame fr = make_frame(g, dp, (G + ngf - 1) / ngf);
   const seis::TimeConsts k = seis::make_consts(dt, h);
   hipStream_t s = (hipStream_t)stream;
@@ -1088,9 +1088,9 @@ int seis_habc_backward(const float* vp, const float* b, const float* wavelet, in
   if (dp.x1 <= dp.x0 || dp.z1 <= dp.z0) dp = Deep{0, 0, 0, 0};  // no deep cells
   const Grid gd{dp.z1 - dp.z0, dp.x1 - dp.x0, 0, (int64_t)(dp.z1 - dp.z0) * (dp.x1 - dp.x0)};
   const TileMap tmd = make_tiles(gd, VX, kHabcRZ, G);
-  const int ngf = std::min(G, frame_groups(nz, nx, G, kFrameGroups));
+  const int ngf = frame_groups(nz, nx, G, S);
   const Frame fr = make_frame(g, dp, (G + ngf - 1) / ngf, true);
-  const int ngb = std::min(G, std::min(kBandGroups, 2 * ngf));
+  const int ngb = even_share(G, std::min(kBandGroups, 2 * ngf));
   const TileMap tmb = band_tiles(g, dp, kBandVX, (G + ngb - 1) / ngb);
   const TileMap tms = side_tiles(g, dp, (G + ngb - 1) / ngb);
   SEIS_CHECK_ARG(tms.per == 0 || (dp.x0 <= kLanes && (int)nx - dp.x1 <= kLanes),

@@ -297,7 +297,7 @@ int seis_habc_march_forward(const float* vp, const float* b, const float* wavele
   const HabcCtx hc{seis::make_grid(nz, nx, npml, multiple != 0), multiple ? 1 : 0, dt, h};
   const Grid& g = hc.g;
   const int S = shots_per_group, G = (int)((B + S - 1) / S);
-  const int ngf = frame_groups(nz, nx, G, 4);
+  const int ngf = frame_groups(nz, nx, G, S);
   const Deep core = core_of(nz, nx);
   const Plan pl = make_plan(B * (core.z1 - core.z0) * (core.x1 - core.x0), widest(nx), 0, vec_x,
                             rows);
@@ -420,7 +420,7 @@ int seis_habc_march_backward(const float* vp, const float* b, const float* wavel
   const HabcCtx hc{seis::make_grid(nz, nx, npml, multiple != 0), multiple ? 1 : 0, dt, h};
   const Grid& g = hc.g;
   const int S = shots_per_group, G = (int)((B + S - 1) / S);
-  const int ngf = frame_groups(nz, nx, G, 4), ngb = std::min(G, std::min(4, 2 * ngf));
+  const int ngf = frame_groups(nz, nx, G, S), ngb = even_share(G, std::min(4, 2 * ngf));
   const Deep core = core_of(nz, nx);
   const Plan pl = make_plan(B * (core.z1 - core.z0) * (core.x1 - core.x0), widest(nx), 0, vec_x,
                             rows);

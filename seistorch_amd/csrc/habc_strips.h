@@ -126,10 +126,6 @@ __device__ __forceinline__ bool in_deep(int z, int x, const Deep& dp) {
   return z >= dp.z0 && z < dp.z1 && x >= dp.x0 && x < dp.x1;
 }
 
-// Most shot groups per frame thread (see frame_groups): the per-cell set-up of the
-// strips runs once for them.
-constexpr int kFrameGroups = 8;
-
 // Most shot groups per thread of the adjoint's top and bottom bands.
 constexpr int kBandGroups = 8;
 
@@ -860,18 +856,33 @@ TileMap side_tiles(const Grid& g, const Deep& dp, int groups) {
   return m;
 }
 
-// Shot groups per frame thread: enough threads (about 400 thousand) come before
-// sharing the set-up per cell.  us per step, forward / adjoint, of the marching
-// loops' frame launches with groups of two shots: 300 x 500 x 8 1 group 10.7 / 38, 2
-// 11.6 / 41, 4 15.3 / 51; 900 x 2500 x 4 1 group 20.4 / 72, 2 20.0 / 68; x 16 1 group 75.6 /
-// 202, 2 70.1 / 179, 4 69.9 / 167, 8 72.5 / 177.  One step per launch, groups of four
-// shots, all in one thread and by this rule: 242 x 300 x 7 13.1 / 39.7 and 10.0 / 35.1,
-// 300 x 500 x 8 15.1 / 46.7 and 11.3 / 38.2, 313 x 344 x 13 20.1 / 60.8 and 12.3 / 42.6.
+// n of G groups per thread at most, evened out over the threads that this takes.
+inline int even_share(int G, int n) {
+  const int parts = (G + n - 1) / n;
+  return (G + parts - 1) / parts;
+}
+
+// Shot groups (of S shots) per frame thread: enough threads come before sharing the
+// set-up per cell, which weighs more in smaller groups.  Powers of two (three groups
+// split 16 unevenly, and bands of six); three groups in one thread rather than in two
+// and one.  us per step, forward / adjoint, with 1 / 2 / 4 groups per thread (threads
+// with one):
+//   one step per launch, S = 4: 300 x 500 x 8 (170 10^3) 16 / 44, 19 / 52; 900 x 1200 x
+//   8 (445 10^3) 27.6 / 67.3, 28.7 / 70.7; 300 x 500 x 32 (680 10^3) 25.0 / 66.8, 26.1 /
+//   65.7, 33 / 92; 500 x 700 x 32 (1.0 10^6) 35.2 / 103, 33.4 / 100, 40 / 105; 164 x 164 x
+//   200 (1.7 10^6) 34 / 129, 36 / 126, 37 / 138; 450 x 450 x 128 (3.1 10^6) 108 / 304, 103 /
+//   283, 102 / 271 (8 groups: 109 / 286); S = 2: 553 x 692 x 3 (260 10^3) 13.9 / 40.4, 14.3 /
+//   42.1; 900 x 1500 x 3 (510 10^3) 20.2 / 52.0, 18.4 / 49.8;
+//   the marching loops, S = 2: 900 x 1500 x 3 18.1 / 48.2, 18.3 / 50.4; 1800 x 1700 x 4 (740
+//   10^3) 31.7 / 87.0, 30.7 / 86.6; 1500 x 1700 x 5 (1.0 10^6) 34.1 / 104, 34.7 / 90.7, all
+//   three 31.5 / 90.1; 600 x 650 x 32 (2.1 10^6) 40 / 125, 36 / 114, 37 / 110.
 // The adjoint's bands, whose set-up is longer, take twice as many: 451 x 877 x 4 37.2
 // for 39.1, 300 x 500 x 8 37.7 for 38.7.
-inline int frame_groups(int64_t nz, int64_t nx, int G, int most) {
-  const int64_t threads = 2 * (kW + 3) * (nz + nx) * G;
-  return (int)std::max<int64_t>(1, std::min<int64_t>(most, (threads + 200000) / 400000));
+inline int frame_groups(int64_t nz, int64_t nx, int G, int S) {
+  const int64_t threads = 2 * (kW + 3) * (nz + nx) * G, line = S <= 2 ? 270000 : 400000;
+  const int64_t q = (threads + line / 2) / line;
+  if (G == 3 && q >= 3) return 3;
+  return even_share(G, q >= 8 ? 4 : q >= 2 ? 2 : 1);
 }
 
 int habc_check(int64_t B, int64_t nz, int64_t nx, float dt, float h, int S) {
