@@ -62,15 +62,20 @@ def _time_step_backward_multiple(*args, **kwargs):
 
 # ----------------------------------------------------------------- fused loop
 
+CORE_MARGIN = 57  # cells between the grid's edges and the part that marches
+
+
 def _march_fits(B, nz, nx):
     """Whether the marching loops take the grid and pay for their launches of the
-    frame's steps: beyond what the last-level cache holds of five fields (about 12
-    10^6 cells).  us per step, forward / adjoint, one step per launch and marching:
-    164 x 164 x 1 shot 6.3 / 24 and 6.5 / 25, 900 x 2500 x 1 10.7 / 38 and 11.7 / 38, 313
-    x 344 x 13 12.3 / 43 and 11.6 / 45, 300 x 500 x 40 23 / 72 and 25 / 72, 900 x 2500 x 4
-    22 / 64 and 20 / 68, x 6 34 / 124 and 31 / 87, x 8 38 / 145 and 40 / 105, x 16 109 /
-    263 and 70 / 168."""
-    return B >= 4 and B * nz * nx >= 12000000 and bool(_lib.load().seis_habc_march_fits(nz, nx))
+    frame's steps: from 8 10^6 cells away from the edges on.  us per step, forward +
+    adjoint, one step per launch and marching (10^6 such cells): 900 x 1500 x 3 (3.3) 71 and
+    69, 1500 x 2500 x 2 (6.6) 87 and 86, 700 x 1500 x 9 (7.3) 112 and 127, 450 x 450 x 64 (7.2)
+    162 and 174, 250 x 250 x 200 (3.7) 208 and 232, 600 x 650 x 32 (8.3) 141 and 145, 3000 x 3000 x
+    1 (8.3) 122 and 103, 900 x 1300 x 10 (9.3) 135 and 135, 700 x 1000 x 20 (10.4) 168 and 157,
+    1500 x 1700 x 5 (11) 171 and 123, 450 x 450 x 128 (14) 373 and 328, 2500 x 2500 x 3 (17) 252
+    and 149, 900 x 2500 x 16 (30) 389 and 257."""
+    core = B * max(nz - 2 * CORE_MARGIN, 0) * max(nx - 2 * CORE_MARGIN, 0)
+    return core >= 8000000 and bool(_lib.load().seis_habc_march_fits(nz, nx))
 
 
 def _march_rows(rec_flat, nz, nx):
