@@ -241,11 +241,10 @@ def _march_forward(bufs, work, vp, d, wavelet, src_zx, rec_flat, rows, rec, ring
 
 
 def _march_backward(bufs, work, vp, d, wavelet, src_zx, rec_flat, rows, grad_rec, ring, snaps, K,
-                    u_a, u_b, B, dt, h, multiple, shape=(0, 0, 0)):
+                    u_a, u_b, grad, B, dt, h, multiple, shape=(0, 0, 0)):
     """The gradient with up to four reverse steps per launch; bufs: two more
     forward fields, four adjoint fields and the shots' gradients."""
     nz, nx = vp.shape
-    grad = torch.empty_like(vp)
     _lib.call("seis_acoustic_march_backward", _lib.ptr(vp), _lib.ptr(d), _lib.ptr(wavelet),
               wavelet.shape[0], _lib.ptr(src_zx), _lib.ptr(rec_flat), rec_flat.shape[0],
               _lib.ptr(rows[0]), rows[1], _lib.ptr(grad_rec), _lib.ptr(ring), _lib.ptr(snaps),
@@ -253,7 +252,6 @@ def _march_backward(bufs, work, vp, d, wavelet, src_zx, rec_flat, rows, grad_rec
               _lib.ptr_array([u_a, u_b, bufs[0], bufs[1]]), _lib.ptr_array(bufs[2:6]),
               _lib.ptr(bufs[6]), _lib.ptr(grad), B, nz, nx, dt, h, NPML, int(multiple), *shape,
               _lib.stream_of(vp))
-    return grad
 
 
 class AcousticLoop(torch.autograd.Function):
@@ -295,7 +293,6 @@ class AcousticLoop(torch.autograd.Function):
         if two_step and not two_step_adjoint and all(v is None for v in shape) \
                 and _march_fits(B, nz, nx, need_grad, multiple):
             rows = _march_rows(rec_flat, nz, nx)
-        bufs = _march_buffers(vp, rows, R, B, 4, False) if rows and illum is None else None
         rec = torch.empty((nt, R), device=vp.device, dtype=torch.float32)
         ring = None
         if need_grad and nt > 1:
@@ -311,6 +308,8 @@ class AcousticLoop(torch.autograd.Function):
             n_snap = int(_lib.load().seis_snapshot_count(nt, K))
             if n_snap > 0:
                 snaps = torch.empty((n_snap, 2, B, nz, nx), device=vp.device, dtype=torch.float32)
+        # after what every loop needs, so that None means that only the others fit
+        bufs = _march_buffers(vp, rows, R, B, 4, False) if rows and illum is None else None
         if bufs is not None:
             u_a, u_b = _march_forward(*bufs, vp, d, wavelet, src_zx, rec_flat, rows, rec, ring,
                                       snaps, K, B, dt, h, multiple)
@@ -365,15 +364,15 @@ class AcousticLoop(torch.autograd.Function):
         R = rec_flat.shape[0]
         G = (B + S - 1) // S
         grad_rec = grad_rec.contiguous().to(torch.float32)
+        grad = torch.empty_like(vp)
         bufs = _march_buffers(vp, rows, R, B, 7, True) if rows else None
         if bufs is not None:
-            grad = _march_backward(*bufs, vp, d, wavelet, src_zx, rec_flat, rows, grad_rec, ring,
-                                   snaps, K, u_a, u_b, B, dt, h, multiple)
+            _march_backward(*bufs, vp, d, wavelet, src_zx, rec_flat, rows, grad_rec, ring, snaps,
+                            K, u_a, u_b, grad, B, dt, h, multiple)
             return (grad,) + (None,) * 15
         mu_a = torch.empty_like(u_a)
         mu_b = torch.empty_like(u_a)
         gpart = torch.empty((G, nz, nx), device=vp.device, dtype=torch.float32)
-        grad = torch.empty_like(vp)
         extra = [None] * 5  # u_c, u_d, mu_c, mu_d, rec_map of the two-step adjoint
         if two_step_adjoint and nt >= 4 and ring is not None:
             ok, rmap = shared_receiver_map(rec_flat, B, nz, nx)

@@ -62,6 +62,7 @@ def _time_step_backward_multiple(*args, **kwargs):
 
 # ----------------------------------------------------------------- fused loop
 
+MARCH_SHOTS = 2   # shots per group of the marching loops' frame steps
 CORE_MARGIN = 57  # cells between the grid's edges and the part that marches
 
 
@@ -88,13 +89,16 @@ def _march_rows(rec_flat, nz, nx):
     return (row_slot, slots) if slots <= max(MARCH_ROWS, nz // MARCH_ROW_SHARE) else None
 
 
-def _march_buffers(vp, rows, R, B, n_fields):
-    """n_fields (B, nz, nx) buffers and the workspace of a marching loop, or None
-    when they do not fit (the one-step loops need fewer)."""
+def _march_buffers(vp, rows, R, B, n_fields, groups=0):
+    """n_fields (B, nz, nx) buffers, the gradient planes of the shot groups if any, and
+    the workspace of a marching loop, or None when they do not fit (the one-step
+    loops need fewer)."""
     nz, nx = vp.shape
     n = int(_lib.load().seis_habc_march_workspace(B, nz, nx, rows[1], R))
     try:
         bufs = [torch.empty((B, nz, nx), device=vp.device) for _ in range(n_fields)]
+        if groups:
+            bufs.append(torch.empty((groups, nz, nx), device=vp.device))
         return bufs, torch.empty(n, device=vp.device)
     except torch.cuda.OutOfMemoryError:
         return None
@@ -116,19 +120,17 @@ def _march_forward(bufs, work, vp, b, wavelet, src_zx, rec_flat, rows, rec, ring
 
 
 def _march_backward(bufs, work, vp, b, wavelet, src_zx, rec_flat, rows, grad_rec, ring, snaps, K,
-                    u_a, u_b, gpart, B, dt, h, multiple, S, shape=(0, 0)):
+                    u_a, u_b, grad, B, dt, h, multiple, S, shape=(0, 0)):
     """The gradient with up to four reverse steps per launch; bufs: two more
-    forward fields, five adjoint fields and the shots' gradients."""
+    forward fields, five adjoint fields, the shots' gradients and the shot groups'."""
     nz, nx = vp.shape
-    grad = torch.empty_like(vp)
     _lib.call("seis_habc_march_backward", _lib.ptr(vp), _lib.ptr(b), _lib.ptr(wavelet),
               wavelet.shape[0], _lib.ptr(src_zx), _lib.ptr(rec_flat), rec_flat.shape[0],
               _lib.ptr(rows[0]), rows[1], _lib.ptr(grad_rec), _lib.ptr(ring), _lib.ptr(snaps),
               K if snaps is not None else 0, _lib.ptr(work),
               _lib.ptr_array([u_a, u_b, bufs[0], bufs[1]]), _lib.ptr_array(bufs[2:7]),
-              _lib.ptr(bufs[7]), _lib.ptr(gpart), _lib.ptr(grad), B, nz, nx, dt, h, NPML,
+              _lib.ptr(bufs[7]), _lib.ptr(bufs[8]), _lib.ptr(grad), B, nz, nx, dt, h, NPML,
               int(multiple), S, *shape, _lib.stream_of(vp))
-    return grad
 
 
 class HabcLoop(torch.autograd.Function):
@@ -154,10 +156,7 @@ class HabcLoop(torch.autograd.Function):
             from .. import autotune
             tuned = autotune.lookup("habc", B, nz, nx)
             shots_per_group = tuned[0] if tuned else None
-        bufs = _march_buffers(vp, rows, R, B, 5) if rows else None
-        # the marching loops' frame steps in pairs of shots
-        S = min(B, 2) if bufs else int(shots_per_group or default_shots_per_group(B))
-        u = None if bufs else [torch.empty((B, nz, nx), device=vp.device) for _ in range(3)]
+        S = int(shots_per_group or default_shots_per_group(B))
         rec = torch.empty((nt, R), device=vp.device)
         ring = snaps = None
         K = 0
@@ -170,11 +169,14 @@ class HabcLoop(torch.autograd.Function):
             n_snap = int(_lib.load().seis_snapshot_count(nt, K))
             if n_snap > 0:
                 snaps = torch.empty((n_snap, 2, B, nz, nx), device=vp.device)
+        # after what every loop needs, so that None means that only one step fits
+        bufs = _march_buffers(vp, rows, R, B, 5) if rows else None
         if bufs is not None:
             u = _march_forward(*bufs, vp, b, wavelet, src_zx, rec_flat, rows, rec, ring, snaps, K,
-                               B, dt, h, multiple, S)
+                               B, dt, h, multiple, min(B, MARCH_SHOTS))
             bufs = None
         else:
+            u = [torch.empty((B, nz, nx), device=vp.device) for _ in range(3)]
             _lib.call("seis_habc_forward", _lib.ptr(vp), _lib.ptr(b), _lib.ptr(wavelet), nt,
                       _lib.ptr(src_zx), _lib.ptr(rec_flat), R, _lib.ptr(rec), _lib.ptr(ring),
                       _lib.ptr(snaps), K, _lib.ptr(illum), _lib.ptr(u[0]), _lib.ptr(u[1]),
@@ -197,17 +199,15 @@ class HabcLoop(torch.autograd.Function):
         nz, nx = vp.shape
         nt = wavelet.shape[0]
         R = rec_flat.shape[0]
-        G = (B + S - 1) // S
         grad_rec = grad_rec.contiguous().float()
-        bufs = _march_buffers(vp, rows, R, B, 8) if rows else None
+        grad = torch.empty_like(vp)
+        bufs = _march_buffers(vp, rows, R, B, 8, -(-B // MARCH_SHOTS)) if rows else None
         if bufs is not None:
-            gpart = torch.empty((G, nz, nx), device=vp.device)
-            grad = _march_backward(*bufs, vp, b, wavelet, src_zx, rec_flat, rows, grad_rec, ring,
-                                   snaps, K, u_a, u_b, gpart, B, dt, h, multiple, S)
+            _march_backward(*bufs, vp, b, wavelet, src_zx, rec_flat, rows, grad_rec, ring, snaps,
+                            K, u_a, u_b, grad, B, dt, h, multiple, min(B, MARCH_SHOTS))
             return (grad,) + (None,) * 11
         lam = [torch.empty_like(u_a) for _ in range(3)]
-        gpart = torch.empty((G, nz, nx), device=vp.device)
-        grad = torch.empty_like(vp)
+        gpart = torch.empty((-(-B // S), nz, nx), device=vp.device)
         _lib.call("seis_habc_backward", _lib.ptr(vp), _lib.ptr(b), _lib.ptr(wavelet), nt,
                   _lib.ptr(src_zx), _lib.ptr(rec_flat), R,
                   _lib.ptr(grad_rec), _lib.ptr(ring), _lib.ptr(snaps),
