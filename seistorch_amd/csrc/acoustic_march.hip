@@ -286,6 +286,15 @@ int check_march(int64_t B, int64_t nz, int64_t nx, float dt, float h, int64_t nt
   return 0;
 }
 
+// A lane (of up to four cells) may hold one of the ring's columns only.
+int check_ring(int64_t nz, int64_t nx, int32_t npml, int64_t ring_len) {
+  SEIS_CHECK_ARG(ring_len > 0, "grid %lld x %lld has no interior inside npml=%d", (long long)nz,
+                 (long long)nx, npml);
+  SEIS_CHECK_ARG(nx - 2 * npml - 1 >= 4, "interior of %lld x %lld too small", (long long)nz,
+                 (long long)nx);
+  return 0;
+}
+
 // One problem's operands.
 struct Problem {
   const float *vp, *d, *wavelet;
@@ -535,9 +544,8 @@ int final_grad(const AdjRun& r, float* grad, hipStream_t s) {
 
 int check_adjoint(int64_t nz, int64_t nx, int64_t nt, int32_t npml, int32_t multiple,
                   int64_t ring_len, const float* ring) {
-  SEIS_CHECK_ARG(ring_len > 0, "grid %lld x %lld has no interior inside npml=%d", (long long)nz,
-                 (long long)nx, npml);
-  SEIS_CHECK_ARG(nx - 2 * npml - 1 >= 4 && nz - (multiple ? 1 : 2) * npml - 1 >= kMaxT,
+  if (int e = check_ring(nz, nx, npml, ring_len)) return e;
+  SEIS_CHECK_ARG(nz - (multiple ? 1 : 2) * npml - 1 >= kMaxT,
                  "interior of %lld x %lld too small", (long long)nz, (long long)nx);
   SEIS_CHECK_ARG(ring || nt <= 2, "ring storage is required for nt > 2");
   return 0;
@@ -604,6 +612,7 @@ int upload(const std::vector<Item>& items, Item* table, hipStream_t s) {
 }
 
 constexpr int kShapeCols = 6;  // nz, nx, B, nt, R, slots
+constexpr int64_t kMaxProblems = (int64_t)1 << 20;
 
 struct Batch {
   std::vector<Problem> p;
@@ -618,7 +627,7 @@ int make_batch(Batch& b, int64_t n, const int64_t* shape, const float* dt_h, con
                const float* d, const float* wavelet, const int32_t* src, const int64_t* rec_flat,
                const int32_t* row_slot, bool rings, float* snaps, int32_t snap_every, float* work,
                int32_t npml, bool adjoint, int32_t vec_x, int32_t rows) {
-  SEIS_CHECK_ARG(n >= 1 && n <= 1 << 20 && shape && dt_h, "bad batch of %lld", (long long)n);
+  SEIS_CHECK_ARG(n >= 1 && n <= kMaxProblems && shape && dt_h, "bad batch of %lld", (long long)n);
   SEIS_CHECK_ARG(snap_every >= 0, "snap_every %d", snap_every);
   int64_t model = 0, wav = 0, so = 0, ro = 0, oo = 0, ri = 0, sn = 0, fo = 0, sl = 0;
   for (int64_t i = 0; i < n; ++i) {
@@ -640,8 +649,8 @@ int make_batch(Batch& b, int64_t n, const int64_t* shape, const float* dt_h, con
     p.g = seis::make_grid(nz, nx, npml, false);
     p.k = seis::make_consts(dt_h[2 * i], dt_h[2 * i + 1]);
     p.ring_len = rings ? seis_ring_len(nz, nx, npml, 0) : 0;
-    SEIS_CHECK_ARG(!rings || p.ring_len > 0, "grid %lld x %lld has no interior inside npml=%d",
-                   (long long)nz, (long long)nx, npml);
+    if (rings)
+      if (int e = check_ring(nz, nx, npml, p.ring_len)) return e;
     p.snaps = snaps ? snaps + sn : nullptr;
     p.snap_every = snap_every;
     p.w = carve(work ? work + b.floats : nullptr, B, nz, nx, q[5], R, adjoint);
@@ -720,8 +729,8 @@ int seis_acoustic_march_forward(const float* vp, const float* d, const float* wa
   if (int e = check_fields(fields)) return e;
   SEIS_CHECK_ARG(!snaps || snap_every > 0, "snapshots need snap_every > 0");
   const int64_t ring_len = ring ? seis_ring_len(nz, nx, npml, multiple) : 0;
-  SEIS_CHECK_ARG(!ring || ring_len > 0, "grid %lld x %lld has no interior inside npml=%d",
-                 (long long)nz, (long long)nx, npml);
+  if (ring)
+    if (int e = check_ring(nz, nx, npml, ring_len)) return e;
   const Grid g = seis::make_grid(nz, nx, npml, multiple != 0);
   const TimeConsts k = seis::make_consts(dt, h);
   const Plan p = make_plan(B * nz * nx, widest(nx), steps, vec_x, rows);
@@ -803,8 +812,12 @@ int seis_acoustic_march_backward(const float* vp, const float* d, const float* w
 
 int64_t seis_acoustic_march_batch_workspace(int64_t n, const int64_t* shape, int32_t snap_every,
                                             int32_t adjoint) {
+  if (n < 1 || n > kMaxProblems || !shape) {
+    seis::set_error("bad batch of %lld", (long long)n);
+    return -1;
+  }
   Batch b;
-  std::vector<float> ones(2 * (size_t)std::max<int64_t>(n, 0), 1.0f);
+  std::vector<float> ones(2 * (size_t)n, 1.0f);
   if (make_batch(b, n, shape, ones.data(), nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
                  false, nullptr, snap_every, nullptr, 0, adjoint != 0, 0, 0))
     return -1;
