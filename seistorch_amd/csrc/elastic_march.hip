@@ -96,7 +96,7 @@ __device__ __forceinline__ void el_special(Const<ElParams> p0, int b, const Lane
 template <int T, int VX, bool EDGE, bool RINGCOLS>
 __device__ __forceinline__ void el_march_strip(const ElParams& p, Const<ElParams> pc, int b,
                                                int strip, int seg) {
-  constexpr int kAhead = 2;
+  constexpr int kAhead = kRowsAhead;
   const Lane l = make_lane<T, VX>(strip, p.sp, p.g.nx);
   const int64_t plane = p.g.plane, off = (int64_t)b * plane;
   const int nz = p.g.nz;

@@ -92,7 +92,9 @@ inline int zero(float* p, int64_t n, hipStream_t s) {
 
 inline int64_t pad64(int64_t n) { return (n + 63) / 64 * 64; }
 
-inline int aux_blocks(int64_t n) { return (int)std::min<int64_t>((n + kThreads - 1) / kThreads, 512); }
+inline int aux_blocks(int64_t n) {
+  return (int)std::min<int64_t>((n + kThreads - 1) / kThreads, 512);
+}
 
 inline int64_t split_blocks(const Split& sp, int64_t B) {
   const int64_t units = (int64_t)sp.strips * sp.segs * sp.group * ((B + sp.group - 1) / sp.group);
@@ -145,9 +147,10 @@ __global__ __launch_bounds__(kThreads) void k_sources(Sources so) { fill_sources
 constexpr int kShotGroup = 8;
 
 constexpr int kMaxT = kMaxSteps;
-// Steps of the next launch when `left` remain to the next boundary: the
-// remainder first, so that the launch that ends at the boundary takes at
-// least two steps (and can write both fields of a snapshot) unless left == 1.
+// Steps of the next launch when `left` remain to the next boundary: the remainder
+// first, so that the launch that ends at the boundary takes all max_t steps (and can
+// write both fields of a snapshot).  With fewer left, the last launch may be a single
+// step, and the pair's first field is copied.
 inline int next_steps(int64_t left, int max_t) {
   const int64_t r = left % max_t;
   if (r == 0) return max_t;
