@@ -385,21 +385,31 @@ ElWork carve_el(float* base, int64_t B, int64_t nx, int64_t slots, int64_t R) {
 
 // Launch shape; 0 = automatic.  Three steps per launch at every size (two were
 // slower throughout; four would need the coefficients of five rows).  Short segments
-// give the most waves, long ones recompute least; us per step with (cells per lane,
-// rows), the best and the next: 164 x 164 x 1 shot (1, 4) 5.0, (1, 8) 6.4; 300 x 500 x
-// 2 (1, 4) 5.4, (1, 8) 6.5; 451 x 877 x 4 (1, 16) 10.3, (1, 12) 11.2; 300 x 500 x 16 (1,
-// 12) 10.6, (1, 8) 11.6; 700 x 1900 x 8 (2, 32) 46.9, (1, 32) 50.1; 900 x 2500 x 16 (2, 32)
-// 154, (1, 32) 171.  The last two are bound by HBM (40 bytes per cell and launch, 29
-// us per step at the rate of a large copy for 700 x 1900 x 8) and by the issue of
-// vector instructions; one step per launch, with launches for sources and records,
-// took 21 us at 451 x 877 x 4 and 116 us at 700 x 1900 x 8.
+// give the most waves, long ones recompute least.  us per step with segments of 4 / 8 /
+// 12 / 16 rows, one cell per lane:
+//   0.03 10^6 cells, 164 x 164 x 1 shot 5.0 / 6.3 / 7.2 / 8.0; 0.6, 300 x 500 x 4 6.9 / 7.3 /
+//   8.2 / 9.1;
+//   0.9, 800 x 1100 x 1 8.6 / 8.0 / 8.4 / 9.2; 300 x 500 x 6 7.8 / 7.6 / 8.3 / 9.1; 1.2, 300 x
+//   500 x 8 10.3 / 8.2 / 9.1 / 9.1; 1.3, 700 x 900 x 2 10.3 / 8.9 / 9.7 / 9.2;
+//   1.5, 500 x 601 x 5 12.2 / 10.9 / 10.9 / 10.4; 1.6, 451 x 877 x 4 13.4 / 11.9 / 11.8 / 10.9;
+//   1.8, 600 x 1000 x 3 12.9 / 10.1 / 11.1 / 10.6; 1200 x 1500 x 1 13.0 / 11.3 / 10.7 / 10.1; 300
+//   x 500 x 12 16.5 / 12.3 / 11.3 / 12.4; 1.7, 164 x 164 x 64 14.2 / 9.7 / 9.7 / 10.7;
+//   2.4, 300 x 500 x 16 16.9 / 12.6 / 11.5 / 12.6; 2.7, 900 x 1500 x 2 17.4 / 13.2 / 12.3 / 11.8;
+//   4.0, 500 x 1000 x 8 24 / 17.3 / 16.6 / 17.5; 4.3, 900 x 1200 x 4 26 / 18.7 / 17.4 / 16.5;
+// and with 12 / 32 rows, 32 with two cells per lane: 4.9, 1300 x 1900 x 2 23.3 / 22.6, 27.5;
+// 5.8, 800 x 900 x 8 22.9 / 24.4, 25.4; 7.2, 1200 x 1501 x 4 39.8 / 34.4; 700 x 1900 x 8 50.1,
+// 46.9 (32 rows); 900 x 2500 x 16 171, 154.  The last two are bound by HBM (40 bytes per
+// cell and launch, 29 us per step at the rate of a large copy for 700 x 1900 x 8) and by
+// the issue of vector instructions; one step per launch, with launches for sources and
+// records, took 21 us at 451 x 877 x 4 and 116 us at 700 x 1900 x 8.
 struct ElShape {
   int vx, rows;
 };
 
 ElShape el_shape(int64_t n, int64_t nx, int32_t vec_x, int32_t rows) {
   ElShape s{1, 32};
-  if (n < 1000000) s.rows = 4;
+  if (n < 750000) s.rows = 4;
+  else if (n < 1400000) s.rows = 8;
   else if (n < 2000000) s.rows = 16;
   else if (n < 5000000) s.rows = 12;
   else if (nx % 2 == 0) s.vx = 2;
