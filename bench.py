@@ -25,19 +25,40 @@ HELD_OUT_SEED = 20240611  # generator stream of the preconditioner's held-out pa
 HBM_PEAK = 8.0e12  # B/s, MI355X
 # algorithmic bytes per cell-update of each timed kernel (fields touched once
 # per step, damping/coefficients read once per cell)
-# (k_fwd2 advances two steps per launch, k_march_fwd and k_march_adj four, the
-# HABC loops four with their frame's steps and k_el_fwd three: their figures are
-# per cell of a launch; the batched marching kernels' are per cell-update)
-BYTES_PER_CELL = {"k_fwd": 16.0, "k_bwd": 36.0, "k_fwd2": 32.0, "k_bwd2": 72.0,
-                  "k_march_fwd": 16.0, "k_march_adj": 40.0,
-                  "k_habc_fwd": 16.0, "k_habc_adj": 40.0,
-                  "k_el_fwd": 43.0, "k_el_bwd": 116.0,
-                  "k_march_fwd_batch": 4.0, "k_march_adj_batch": 10.0}
+BYTES_PER_CELL = {"k_fwd": 16.0, "k_bwd": 36.0, "k_fwd2": 16.0, "k_bwd2": 36.0,
+                  "k_habc_fwd": 16.0, "k_habc_adj": 36.0, "k_el_fwd": 52.0, "k_el_bwd": 116.0}
 KERNEL_IDS = {"acoustic": (("k_fwd", 0), ("k_bwd", 1), ("k_fwd2", 8), ("k_bwd2", 9),
                            ("k_march_fwd", 11), ("k_march_adj", 12)),
               "habc": (("k_habc_fwd", 4), ("k_habc_adj", 5)),
               "elastic": (("k_el_fwd", 2), ("k_el_bwd", 3)),
               "generator": (("k_march_fwd_batch", 6), ("k_march_adj_batch", 7))}
+
+
+def launch_bytes(name, P):
+    """(algorithmic bytes of one launch that a timing slot covers, its time steps, its
+    kernels, its key in profiles/traffic.json).  The marching loops take four steps
+    (elastic three) per launch; their adjoint reads and writes the forward fields and
+    the gradient (24 bytes) on the undamped interior only, and a marched HABC launch
+    is the core's four steps and the frame's one by one."""
+    N = P["B"] * P["nz"] * P["nx"]
+    if name == "k_march_fwd":
+        return 16.0 * N, 4, name, name
+    if name == "k_march_adj":
+        return 16.0 * N + 24.0 * P["B"] * (P["nz"] - 98) * (P["nx"] - 98), 4, name, name
+    if name in ("k_habc_fwd", "k_habc_adj"):
+        from seistorch_amd.equations2d import acoustic_habc as ah
+        if ah._march_fits(P["B"], P["nz"], P["nx"]):
+            m = 2 * ah.CORE_MARGIN
+            core = P["B"] * (P["nz"] - m) * (P["nx"] - m)
+            if name == "k_habc_fwd":
+                return (16.0 * core + 64.0 * (N - core), 4, "k_core_fwd + 4 k_habc_fwd_deep",
+                        "k_habc_march_fwd")
+            return (40.0 * core + 144.0 * (N - core), 4, "k_core_adj + 4 k_frame_adj",
+                    "k_habc_march_adj")
+    if name == "k_el_fwd":
+        return 43.0 * N, 3, "k_el_march", "k_el_march"
+    steps = 2 if name in ("k_fwd2", "k_bwd2") else 1
+    return BYTES_PER_CELL[name] * N * steps, steps, name, name
 
 
 def parse():
@@ -65,8 +86,9 @@ def parse():
                         "the 64-shot 800x2400 problem")
     p.add_argument("--models", type=int, default=256, help="generator: number of models")
     p.add_argument("--graph", type=int, default=0,
-                   help="generator: 1 records each batched loop into one hipGraph (kernel "
-                        "timing events are then unavailable)")
+                   help="generator: 1 takes the loops with one or two steps per launch, each "
+                        "recorded into one hipGraph (kernel timing events are then "
+                        "unavailable)")
     p.add_argument("--snapshot-every", type=int, default=500,
                    help="generator: field-pair snapshot spacing of the batched adjoint")
     p.add_argument("--pair-models", type=int, default=5000,
@@ -177,10 +199,11 @@ def gradient_step(P):
 
 
 def _launch_shape_json(workload, shape, tune):
-    """The tuned launch shape and the candidates' times for the JSON line."""
+    """The tuned launch shape and the candidates' times for the JSON line (of the
+    elastic loops the adjoint's: the forward marches)."""
     if workload == "elastic":
-        out = {"shots_per_group_forward": shape[0], "shots_per_group_adjoint": shape[1]}
-        times = {f"{k[0]}_S{k[1]}": round(t, 2) for k, t in tune.items()}
+        out = {"shots_per_group_adjoint": shape[1]}
+        times = {f"S{k[1]}": round(t, 2) for k, t in tune.items() if k[0] == "fwd+adj"}
     elif len(shape) == 3:
         out = {"shots_per_group": shape[0], "rows_per_thread": shape[1], "vec_x": shape[2]}
         times = {f"S{a}_rz{b}_vx{c}": round(t, 2) for (a, b, c), t in tune.items()}
@@ -317,8 +340,10 @@ def run_generator(args, dev):
     cells = generator.cell_updates(host)
     print(f"[bench] generator: {len(host)} models, {cells:.3e} cell-updates per propagation, "
           f"built in {time.perf_counter() - t0:.1f} s", file=sys.stderr, flush=True)
-    launch = {}  # the marching loops choose their own launch shape
     use_graph = bool(args.graph)
+    # the four-step loops choose their own launch shape; a graph is of the loops with one
+    # or two steps per launch, which a launch shape asks for
+    launch = dict(shots_per_group=4) if use_graph else {}
     lib = _lib.load()
 
     def step():
@@ -355,9 +380,13 @@ def run_generator(args, dev):
     roof = None
     if not use_graph:
         # per launch the batched kernels cover every running instance; the
-        # algorithmic bytes of all timed launches over their summed duration
+        # algorithmic bytes of all timed launches over their summed duration: per
+        # cell-update 4 for the adjoint fields, 6 more on the undamped interior
         tot_ms, n_launch = kern["k_march_adj_batch"]
-        achieved = BYTES_PER_CELL["k_march_adj_batch"] * cells * args.steps / (tot_ms / 1e3)
+        alg = sum(it["B"] * it["nt"] * (4.0 * it["vp_true"].shape[0] * it["vp_true"].shape[1]
+                                        + 6.0 * (it["vp_true"].shape[0] - 98)
+                                        * (it["vp_true"].shape[1] - 98)) for it in host)
+        achieved = alg * args.steps / (tot_ms / 1e3)
         # measured HBM bytes per cell-update (rocprof counters) x the average
         # cell-updates of one launch
         traffic = None
@@ -370,7 +399,7 @@ def run_generator(args, dev):
         roof = {"bound": "hbm", "kernel": "k_march_adj_batch", "achieved": round(achieved / 1e9, 1),
                 "peak": HBM_PEAK / 1e9, "unit": "GB/s", "frac": round(achieved / HBM_PEAK, 4),
                 "traffic": traffic, "avg_launch_us": round(tot_ms / max(n_launch, 1) * 1e3, 2),
-                "launches": n_launch, "bytes_per_cell_update": BYTES_PER_CELL["k_march_adj_batch"]}
+                "launches": n_launch, "bytes_per_cell_update": round(alg / cells, 2)}
     out = {
         "metric": METRIC, "value": round(value, 3), "unit": "Gcell-updates/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup,
@@ -378,7 +407,8 @@ def run_generator(args, dev):
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32",
         "data": "synthetic (seeded layered/faulted/anomaly models, records from the true models)",
         "config": {"workload": "uneven batch: records + L2-misfit gradient of every model, "
-                               "PML 50, one launch per step over all running models",
+                               "PML 50, all running models in a launch of "
+                               + ("one or two steps" if use_graph else "up to four steps"),
                    "models": len(host), "cell_updates_per_propagation": cells,
                    "nt_range": [min(i["nt"] for i in host), max(i["nt"] for i in host)],
                    "shots_range": [min(i["B"] for i in host), max(i["B"] for i in host)],
@@ -785,7 +815,8 @@ def main():
                                             P["w"], P["src"], P["rec"], P["B"], P["dt"], P["h"],
                                             src_type=("txx", "tzz"), rec_type=("vx", "vz"))
     if shape is not None:
-        print(f"[bench] autotuned launch shape {shape}", file=sys.stderr, flush=True)
+        print(f"[bench] autotuned shots per group of the adjoint: {shape[1]}", file=sys.stderr,
+              flush=True)
     for i in range(args.warmup):
         step_fn(P)
         torch.cuda.synchronize()
@@ -812,12 +843,12 @@ def main():
     dom = max(kern, key=lambda k: kern[k][0])
     tot_ms, n_launch = kern[dom]
     avg_s = tot_ms / max(n_launch, 1) / 1e3
-    alg_bytes = BYTES_PER_CELL[dom] * P["B"] * P["nz"] * P["nx"]
+    alg_bytes, launch_steps, kernels, traffic_key = launch_bytes(dom, P)
     achieved = alg_bytes / avg_s if avg_s > 0 else 0.0
     traffic = None
     tpath = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "traffic.json")
     if os.path.exists(tpath):
-        traffic = json.load(open(tpath)).get(dom)
+        traffic = json.load(open(tpath)).get(traffic_key)
     out = {
         "metric": METRIC, "value": round(value, 3), "unit": "Gcell-updates/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(el / args.steps * 1e3, 2),
@@ -832,11 +863,13 @@ def main():
                    "grid": [P["nz_i"], P["nx_i"]], "padded_grid": [P["nz"], P["nx"]],
                    "shots": P["B"], "nt": P["nt"], "dt": P["dt"], "dx": P["h"],
                    "receivers_per_shot": P["nx_i"], "f_peak_hz": P["fm"]},
-        "roofline": {"bound": "hbm", "kernel": dom, "achieved": round(achieved / 1e9, 1),
+        "roofline": {"bound": "hbm", "kernel": kernels, "achieved": round(achieved / 1e9, 1),
                      "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK, 4), "traffic": traffic,
                      "avg_launch_us": round(avg_s * 1e6, 2), "launches": n_launch,
-                     "bytes_per_cell_update": BYTES_PER_CELL[dom]},
+                     "steps_per_launch": launch_steps, "bytes_per_launch": round(alg_bytes),
+                     "bytes_per_cell_update": round(alg_bytes / launch_steps / P["B"] / P["nz"]
+                                                    / P["nx"], 2)},
         "kernels_ms_total": {k: round(v[0], 2) for k, v in kern.items()},
         "launch_shape": None if shape is None else _launch_shape_json(args.workload, shape, tune),
         "loss": float(loss),

@@ -1,4 +1,4 @@
-"""Launch-shape autotuner for the fused time loops.
+"""Launch-shape autotuner for the fused loops of one or two steps per launch.
 
 For a given equation and problem shape (shots, nz, nx) it times the fused
 forward + adjoint over a short time axis for every candidate launch shape
@@ -6,7 +6,11 @@ forward + adjoint over a short time axis for every candidate launch shape
 the uneven batch, shots_per_group for the elastic and HABC loops -- and keeps
 the fastest.  Results live in a
 process-wide table (and optionally a JSON file), keyed by shape, and
-``propagate`` picks them up when the caller does not fix the launch shape.
+``propagate`` picks them up when the caller does not fix the launch shape and
+these loops run: the elastic adjoint always, HABC where the marching loops do
+not pay, the others where the marching loops do not apply (illumination,
+receivers on many grid rows, memory).  The marching loops, which are faster than
+any shape of these, choose their own launch shapes by size.
 """
 import itertools
 import json

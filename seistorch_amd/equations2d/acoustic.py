@@ -416,13 +416,14 @@ def propagate(vp, d, wavelet, src_zx, rec_flat, B, dt, h, shots_per_group=None,
               two_step_adjoint=False, illum=None, multiple=False, extra_sources=None):
     """Records (nt, R) of B shots; differentiable w.r.t. vp through the adjoint.
 
-    The launch shape -- shots_per_group (1, 2, 4, 8), rows_per_thread
-    (1, 2, 4), vec_x (cells per lane along x: 1, 2, 4, dividing nx) --
-    defaults to the autotuned values for this shape (``seistorch_amd.autotune``),
-    else to fixed defaults.  With none of them given, two_step lets a launch
-    take up to four time steps (reverse steps in the adjoint; receivers on few
-    grid rows, see MARCH_ROWS); with a launch shape it runs two forward time
-    steps per launch.  Records are the same bit for bit in all of them.  two_step_adjoint runs
+    With no launch shape, two_step lets a launch take up to four time steps
+    (reverse steps in the adjoint; receivers on few grid rows, see MARCH_ROWS).
+    A launch shape -- shots_per_group (1, 2, 4, 8), rows_per_thread
+    (1, 2, 4), vec_x (cells per lane along x: 1, 2, 4, dividing nx) -- asks for
+    the loops with two forward time steps per launch and one reverse step; what it
+    leaves open, and all of it where the four-step loops do not apply, is the
+    autotuned shape (``seistorch_amd.autotune``), else a fixed default.  Records are
+    the same bit for bit in all of them.  two_step_adjoint runs
     two reverse steps per adjoint launch (same results up to the order of the
     gradient additions at receiver cells; at present slower than one step per
     launch: its fields of two iterations need ~250 registers per lane).

@@ -135,7 +135,8 @@ def batch_instances(dev_insts, which):
 
 
 def observed(dev_insts, use_graph=True, **launch):
-    """Records of every true model (no gradient state)."""
+    """Records of every true model (no gradient state); use_graph and launch as
+    propagate_batch takes them."""
     from .equations2d.acoustic_batch import propagate_batch
     with torch.no_grad():
         return propagate_batch(batch_instances(dev_insts, "vp_true"), use_graph=use_graph,
